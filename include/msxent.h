@@ -27,9 +27,10 @@
 extern "C" {
 #endif
 
-/* Bytes of device workspace for both calls with this shape and chunk (the backward's probability
- * blocks are n_rows x chunk, chunk rounded up to a multiple of 256 and capped at the vocabulary;
- * the forward uses a prefix of it).  MSD_E_CONFIG for an unsupported shape. */
+/* Bytes of device workspace for both calls with this shape and chunk: the forward's partials (a
+ * prefix), the backward's probability block (n_rows x the chunk the library works in: the caller's,
+ * raised to what fits 256 MiB and capped at the vocabulary) and the f32 partials of grad_h (at
+ * most 64 MiB or one n_rows x d_model, whichever is more).  MSD_E_CONFIG for an unsupported shape. */
 int64_t msd_xent_workspace_bytes(int32_t n_rows, int32_t vocab, int32_t d_model, int32_t chunk);
 
 /* Forward.  loss: device f32 scalar, the mean over rows of lse - target logit; lse: device f32
@@ -45,8 +46,8 @@ int32_t msd_xent_forward(const void* h, const void* weight, const int32_t* targe
  *   grad_h      = (softmax(h W^T) - onehot(targets)) W * g / n_rows
  *   grad_weight = (softmax(h W^T) - onehot(targets))^T h * g / n_rows
  * computed chunk by chunk over the vocabulary (chunk columns at a time, as the reference's loop),
- * with the softmax block rounded to bf16 before its two products; grad_h is summed over the
- * chunks in f32 in vocabulary order.  Deterministic. */
+ * with the softmax block rounded to bf16 before its two products; grad_h is summed in f32, over
+ * fixed ranges of the vocabulary and then over the ranges in order.  Deterministic. */
 int32_t msd_xent_backward(const void* h, const void* weight, const int32_t* targets, const float* lse,
                           const float* grad_loss, int32_t n_rows, int32_t vocab, int32_t d_model,
                           int32_t chunk, void* workspace, void* grad_h, void* grad_weight,

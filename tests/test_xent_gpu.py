@@ -62,6 +62,18 @@ def test_ragged_shapes_and_chunks():
     _against_oracle(1, 77, 128, 4096, seed=2, g=0.5)
 
 
+@pytest.mark.parametrize("N,V,d,chunk", [
+    (65, 257, 128, 100),        # 128-tiles: one row, one id past a tile; token padding to 64
+    (129, 4001, 384, 1000),     # 128-tiles, grad_h split over K with a short last split
+    (1023, 16500, 256, 4096),   # 256-tiles for the logits, 128-tiles for the gradients
+    (4352, 30000, 640, 1000),   # 256-tiles for grad_h with a half-empty last column tile
+    (20000, 7000, 128, 256),    # probability block past its cap: two chunks
+])
+def test_tile_sizes_splits_and_chunks(N, V, d, chunk):
+    """Each tile size of each product, at ragged edges (tolerances as above)."""
+    _against_oracle(N, V, d, chunk, seed=8)
+
+
 def test_peaked_logits():
     """Large logits (h scaled by 40: logit spread ~ 15): the logsumexp stays finite and exact."""
     _against_oracle(513, 3000, 384, 1024, seed=3, h_scale=40.0)

@@ -13,10 +13,10 @@ the reference's backward casts them (model.py:361).
 What runs (``msd_xent_forward`` / ``msd_xent_backward``, ``csrc/xent.hip``): the forward streams
 the whole vocabulary through one MFMA GEMM whose epilogue keeps only each row's running
 (max, sum of exponentials), so no logits are stored; the per-row logsumexp is kept for the
-backward.  The backward runs chunk by chunk over the vocabulary (``chunk_size`` columns, rounded
-up to a multiple of 256): the softmax block minus the one-hot targets, scaled by g / N, is
-formed in bf16 and multiplied into grad_weight (final per chunk) and grad_h (summed over chunks
-in f32).  Differences from the reference: the forward's logits are f32 sums of exact bf16
+backward.  The backward runs chunk by chunk over the vocabulary (at least ``chunk_size`` columns;
+more while a chunk's block stays within 256 MiB): the softmax block minus the one-hot targets,
+scaled by g / N, is formed in bf16 and multiplied into grad_weight (final per chunk) and grad_h
+(f32 partial sums).  Differences from the reference: the forward's logits are f32 sums of exact bf16
 products (the reference's forward runs in the bf16 params dtype), and the backward's softmax
 block is rounded to bf16 before its two products (the reference keeps f32; both end in bf16
 gradients).
