@@ -164,13 +164,13 @@ __device__ __forceinline__ int64_t cache_row(const Rows& r, int m, int p) {
 }
 
 // What mx_gemm_rows does with its final outputs.
-enum Epi { kEpiStore = 0, kEpiSwiglu = 1, kEpiQkv = 2, kEpiResid = 3, kEpiResidNorm = 4 };
+enum Epi { kEpiStore = 0, kEpiSwiglu = 1, kEpiQkv = 2, kEpiResid = 3 };
 // Operands of the fused epilogues.
 struct EpiArgs {
-  uint16_t* act;       // SwiGLU: the down projection's input planes; ResidNorm: the next RMSNorm's
+  uint16_t* act;       // SwiGLU: the down projection's input planes; Resid: the next RMSNorm's (or NULL)
   int64_t act_plane;   // input planes (scale * h); tile order, the lo plane act_plane further
-  const uint16_t* xscale;   // ResidNorm: the next RMSNorm's scales in packed order
-  float* ssq;               // ResidNorm: each row's partial sum of h^2 per column group, [M][N / (16 CT)]
+  const uint16_t* xscale;   // Resid: the next RMSNorm's scales in packed order
+  float* ssq;               // Resid: each row's partial sum of h^2 per column group, [M][N / (16 CT)]
   const float* rope;   // QKV: RoPE table, rows, cache and the f32 q/k/v rows (as mx_qkv_fin)
   Rows rows;
   uint16_t* kc;
@@ -317,36 +317,72 @@ __device__ __forceinline__ void qkv_pair(float s0, float s1, float c, float sg, 
   }
 }
 
+// Two f32 values as hi/lo parts, packed (a in the low halves; v_cvt_pk_bf16_f32 rounds to nearest even).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  hi = pack2(a, b);
+  lo = pack2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
+}
+
+// Four outputs of the packed q/k/v rows col .. col + 3 (col a multiple of 4): qkv_pair for both pairs
+// with whole-run stores.  rp: the position's RoPE row; q: the row's f32 q/k/v.
+__device__ __forceinline__ void qkv_quad(f32x4 v, const float* rp, int col, int H, int KV, float* q, uint16_t* kc,
+                                         uint16_t* vc, int64_t pool, int64_t crow) {
+  const int head = col / kDh, rr = col % kDh;
+  q += head * kDh;
+  if (head >= H + KV) {   // v: four consecutive dims
+    *reinterpret_cast<f32x4*>(q + rr) = v;
+    *reinterpret_cast<uint2*>(vc + (int64_t(head - H - KV) * pool + crow) * kDh + rr) =
+        make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+    return;
+  }
+  const int ri = rr >> 1;   // pairs: dims ri, ri + 32 and ri + 1, ri + 33
+  const f32x2 c = *reinterpret_cast<const f32x2*>(rp + ri), s = *reinterpret_cast<const f32x2*>(rp + kDh / 2 + ri);
+  const f32x2 x = {v[0] * c[0] - v[1] * s[0], v[2] * c[1] - v[3] * s[1]};
+  const f32x2 y = {v[0] * s[0] + v[1] * c[0], v[2] * s[1] + v[3] * c[1]};
+  *reinterpret_cast<f32x2*>(q + ri) = x;
+  *reinterpret_cast<f32x2*>(q + ri + kDh / 2) = y;
+  if (head >= H) {
+    uint16_t* cp = kc + (int64_t(head - H) * pool + crow) * kDh;
+    *reinterpret_cast<uint32_t*>(cp + ri) = pack2(x[0], x[1]);
+    *reinterpret_cast<uint32_t*>(cp + ri + kDh / 2) = pack2(y[0], y[1]);
+  }
+}
+
 // C = A W^T for many rows: a workgroup owns 16 RT rows x 16 CT columns over the whole of K, so it
-// streams CT * 16 complete weight rows (contiguous in memory) and writes final outputs (no split-K
-// partials); with RT = 2 every weight tile it loads serves 32 rows, and the last column group may
-// be short (ragged: N / 16 need not be a multiple of CT).  The four waves take interleaved
-// 32-wide K steps (wave w: steps w, w + 4, ...) with P steps of loads in flight, and add their
-// tiles through LDS in wave order, so the result is deterministic.  Tiles are dealt XCD-aware:
-// every row tile of a column tile runs on one XCD (workgroup b on XCD b mod 8), which then fetches
-// that column tile's weights into its L2 once.  AM: the A operand as bf16 hi/lo rows (0) or tiles (1) as for mx_gemm, or (2) RMSNorm
-// folded in (model.py:94-98): A = the hi/lo tiles of scale * h that the previous projection's
-// epilogue wrote (kEpiResidNorm), and every output divided by sqrt(mean(h^2) + 1e-5), the sum of
+// streams 16 CT complete weight rows (contiguous in memory), every weight tile it loads serves
+// 16 RT rows, and it writes final outputs (no split-K partials).  The last column group may be
+// short (N / 16 need not be a multiple of CT).  Its NW waves each hold the whole output tile and
+// take interleaved 32-wide K steps (wave w: steps w, w + NW, ...) with P steps of loads in
+// flight; the waves' tiles are added through LDS in wave order, row tile by row tile, so the result
+// is deterministic.  Tiles are dealt XCD-aware: each XCD (workgroup b runs on XCD b mod 8) takes a
+// contiguous range of the tiles, row tiles innermost, so a column group's weights reach its L2 once.
+// AM: the A operand as bf16 hi/lo rows (0) or tiles (1) as for mx_gemm, or (2) RMSNorm folded in
+// (model.py:94-98): A = the hi/lo tiles of scale * h that the previous projection's
+// epilogue wrote (kEpiResid), and every output divided by sqrt(mean(h^2) + 1e-5), the sum of
 // h^2 of each row added up from that epilogue's per-column-group partials.  TW as for mx_gemm.
-// EPI: store the outputs, add them to the residual out (tile order; with kEpiResidNorm also the
+// EPI: store the outputs, add them to the residual out (tile order; with an act plane also the
 // hi/lo tiles of scale * h and the row's partial sum of h^2 for the next RMSNorm), or finish them
 // in place of mx_swiglu_fin / mx_qkv_fin (column pairs per thread, the same arithmetic).
-template <int CT, int P, int AM, bool TW, int EPI, int RT = 1>
-__global__ __launch_bounds__(256) void mx_gemm_rows(GemmArgs g) {
-  static_assert(RT == 1 || (AM >= 1 && TW && (EPI == kEpiSwiglu || EPI == kEpiQkv)),
-                "two row tiles per workgroup: tile-order operands and a pair epilogue");
-  // the waves' partial tiles, element r of lane l's D registers at [r][l]: the epilogue reads
-  // them across lanes contiguously (read as [l][r], 16 bytes apart, they took 2-4 times the LDS
-  // cycles: SQ_LDS_BANK_CONFLICT)
-  __shared__ float red[4][RT][CT][4][64];
-  __shared__ float rrms[16 * RT];   // AM 2: each row's rms
+template <int RT, int CT, int P, int NW, int AM, bool TW, int EPI>
+__global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
+  static_assert(RT == 1 || (AM >= 1 && TW), "several row tiles per workgroup: tile-order operands");
+  // the waves' partial tiles of one row tile, a lane's four outputs as one 16-byte piece (written and
+  // read across lanes contiguously); two buffers, so one barrier per row tile suffices
+  __shared__ f32x4 red[RT > 1 ? 2 : 1][NW][CT][64];
+  __shared__ float rrms[16 * RT];       // AM 2: each row's 1 / rms
+  __shared__ float hs[RT][NW][16];      // kEpiResid: each wave's part of the rows' sums of h^2
   // wave-uniform wave index: the step count and its loop stay scalar (a per-lane loop would copy
   // the accumulators out of and back into the AGPRs around every step)
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = g.N / 16, T = (g.M + 15) / 16, TG = (T + RT - 1) / RT, C = (n16 + CT - 1) / CT;
-  const int b = blockIdx.x, slot = b >> 3;
-  const int t = slot % TG, c = (slot / TG) * 8 + (b & 7);
-  if (c >= C) return;
+  const int xcd = blockIdx.x & 7, per = gridDim.x >> 3, rest = gridDim.x & 7;
+  const int id = xcd * per + min(xcd, rest) + (blockIdx.x >> 3);
+  const int t = id % TG, c = id / TG;
   const int m0 = 16 * RT * t, n0 = 16 * CT * c;
   const int ctn = min(CT, n16 - CT * c);   // column tiles of this group (the last group may be short)
   const int r16 = lane & 15, kq = 8 * (lane >> 4);
@@ -362,146 +398,174 @@ __global__ __launch_bounds__(256) void mx_gemm_rows(GemmArgs g) {
   // element offsets of step ks and of column tile ct
   const int64_t astep = AM >= 1 ? 512 : kBK, wstep = TW ? 512 : kBK;
   const int64_t wtile = TW ? int64_t(S) * 512 : int64_t(16) * g.K;
-  const int ns = (S - wv + 3) / 4;   // K steps of this wave (S >= 4: every wave has one)
+  const int ns = (S - wv + NW - 1) / NW;   // K steps of this wave (possibly none)
   f32x4 acc[RT][CT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // AM 2: the partial sums of h^2 of row 16 rt + tid / 16 (column groups tid % 16 + 16 j),
-  // requested now and added up after the K loop
-  constexpr int kSq = 4;
-  float sq[RT][kSq];
-  if constexpr (AM == 2) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int64_t rrow = min(m0 + 16 * rt + int(threadIdx.x >> 4), g.M - 1);
-#pragma unroll
-      for (int j = 0; j < kSq; ++j) {
-        const int cg = int(threadIdx.x & 15) + 16 * j;
-        sq[rt][j] = g.ssq[rrow * g.nssq + min(cg, g.nssq - 1)];
-      }
-    }
-  }
-  // the residual elements this thread's epilogue updates (one per column tile: row 4 (lane / 16)
-  // + wave of the tile, column 16 ct + lane % 16), requested before the K loop so that the
+  // A thread's outputs are, per column tile ct = wave, wave + NW, ..., row lane % 16 and columns 16 ct
+  // + 4 (lane / 16) .. + 4 (the MFMA's A operand is the weights).  The residual elements it updates
+  // are requested before the K loop (one row tile) or before the row tile's barrier, so that the
   // epilogue does not wait a memory round trip for them (rows past M read row M - 1)
-  float hold[CT];
-  if constexpr (EPI == kEpiResid || EPI == kEpiResidNorm) {
-    const int row = min(m0 + 4 * (lane >> 4) + wv, g.M - 1);
+  constexpr bool kResid = EPI == kEpiResid;
+  constexpr int NI = (CT + NW - 1) / NW;
+  const int orow = lane & 15, ocol = 4 * (lane >> 4);
+  f32x4 hold[NI];
+  auto load_hold = [&](int rt) {
+    if constexpr (kResid) {
+      const int row = min(m0 + 16 * rt + orow, g.M - 1);
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) hold[ct] = g.out[act_index(row, n0 + 16 * ct + (lane & 15), g.N, 0)];
-  }
+      for (int i = 0; i < NI; ++i)
+        hold[i] = *reinterpret_cast<const f32x4*>(
+            g.out + act_index(row, n0 + 16 * min(wv + NW * i, ctn - 1) + ocol, g.N, 0));
+    }
+  };
+  if constexpr (RT == 1) load_hold(0);
   uint4 a[P][RT], al[P][RT], w[P][CT];
   // step i of this wave, clamped to its last: loads stay unconditional, so no wait lands at a
-  // branch join (a column tile past a short group's end reads its last tile)
+  // branch join (a column tile past a short group's end reads its last tile; a wave without steps
+  // reads the first)
   auto load = [&](int p, int i) {
-    const int ks = wv + 4 * min(i, ns - 1);
+    const int ks = min(wv + NW * min(i, ns - 1), S - 1);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+      w[p][ct] = *reinterpret_cast<const uint4*>(wr + min(ct, ctn - 1) * wtile + max(ks, 0) * wstep);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      a[p][rt] = *reinterpret_cast<const uint4*>(ar[rt] + ks * astep);
-      al[p][rt] = *reinterpret_cast<const uint4*>(ar[rt] + g.a_plane + ks * astep);
+      a[p][rt] = *reinterpret_cast<const uint4*>(ar[rt] + max(ks, 0) * astep);
+      al[p][rt] = *reinterpret_cast<const uint4*>(ar[rt] + g.a_plane + max(ks, 0) * astep);
     }
+  };
+  auto mma = [&](int p, bool live) {   // (a step past the end multiplies a zero A fragment)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) w[p][ct] = *reinterpret_cast<const uint4*>(wr + min(ct, ctn - 1) * wtile + ks * wstep);
+    for (int rt = 0; rt < RT; ++rt) {
+      uint4 x = a[p][rt], xl = al[p][rt];
+      if (!live) x = xl = make_uint4(0, 0, 0, 0);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w[p][ct]), as_bf16x8(x), acc[rt][ct], 0, 0, 0);
+        acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w[p][ct]), as_bf16x8(xl), acc[rt][ct], 0, 0, 0);
+      }
+    }
   };
 #pragma unroll
   for (int p = 0; p < P; ++p) load(p, p);
-  // every round runs all P steps (a step past the end multiplies a zero A fragment), so the
-  // accumulators stay in the AGPRs across the loop
-  for (int i0 = 0; i0 < ns; i0 += P) {
+  // AM 2: the sums of h^2 of row 16 rt + tid / 16 (column groups tid % 16 + 16 j), requested
+  // behind the first steps and added up after the K loop
+  constexpr int kSq = 4, NR = (16 * RT * 16 + 64 * NW - 1) / (64 * NW);   // rows per thread
+  float sq[NR][kSq];
+  if constexpr (AM == 2) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const int64_t rrow = min(m0 + int(threadIdx.x >> 4) + 4 * NW * q, g.M - 1);
+#pragma unroll
+      for (int j = 0; j < kSq; ++j) {
+        const int cg = int(threadIdx.x & 15) + 16 * j;
+        sq[q][j] = g.ssq[rrow * g.nssq + min(cg, g.nssq - 1)];
+      }
+    }
+  }
+  // whole rounds of P steps with the next round's loads behind each step, then the last steps
+  // (a load past the end would cost as much traffic as a step)
+  int i0 = 0;
+  for (; i0 + 2 * P <= ns; i0 += P) {
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      const bool live = i0 + p < ns;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        uint4 x = a[p][rt], xl = al[p][rt];
-        if (!live) x = xl = make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x), as_bf16x8(w[p][ct]), acc[rt][ct], 0, 0, 0);
-          acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xl), as_bf16x8(w[p][ct]), acc[rt][ct], 0, 0, 0);
-        }
-      }
+      mma(p, true);
       load(p, i0 + p + P);
     }
   }
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
+  for (int p = 0; p < P; ++p) {
+    mma(p, i0 + p < ns);
+    if (i0 + p + P < ns) load(p, i0 + p + P);
+  }
+  if (i0 + P < ns) {
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int p = 0; p < P - 1; ++p) mma(p, i0 + P + p < ns);
+  }
+  if constexpr (AM == 2) {   // the rows' sums of h^2 over their nssq <= 64 partials, in a fixed order
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[wv][rt][ct][r][lane] = acc[rt][ct][r];
-  if constexpr (AM == 2) {   // row 16 rt + tid / 16's sum of h^2 over its nssq <= 64 partials, in a fixed order
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
+    for (int q = 0; q < NR; ++q) {
       float sum = 0.f;
 #pragma unroll
-      for (int j = 0; j < kSq; ++j) sum += int(threadIdx.x & 15) + 16 * j < g.nssq ? sq[rt][j] : 0.f;
+      for (int j = 0; j < kSq; ++j) sum += int(threadIdx.x & 15) + 16 * j < g.nssq ? sq[q][j] : 0.f;
       sum = sum16_lanes(sum);
-      if ((threadIdx.x & 15) == 0) rrms[16 * rt + (threadIdx.x >> 4)] = sqrtf(sum / float(g.K) + 1e-5f);
+      const int row = int(threadIdx.x >> 4) + 4 * NW * q;
+      if ((threadIdx.x & 15) == 0 && row < 16 * RT) rrms[row] = 1.f / sqrtf(sum / float(g.K) + 1e-5f);
     }
   }
-  __syncthreads();
-  // D layout of a 16 x 16 tile: lane holds rows 4 (lane / 16) + r of column lane % 16
-  if constexpr (EPI == kEpiStore || EPI == kEpiResid || EPI == kEpiResidNorm) {
-    // (one row tile, whole column groups) thread tid holds row 4 (lane / 16) + wave of the tile,
-    // columns 16 ct + lane % 16
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    f32x4(*rd)[CT][64] = red[rt & 1 & (RT - 1)];
+    if constexpr (RT > 1) load_hold(rt);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) rd[wv][ct][lane] = acc[rt][ct];
+    __syncthreads();
+    const int row = m0 + 16 * rt + orow;
+    const bool live = row < g.M;
+    const EpiArgs& ea = g.e;
+    int64_t crow = 0;
+    const float* rp = nullptr;
+    if constexpr (EPI == kEpiQkv) {   // the row's position: cache row and RoPE factors
+      const int p = row_pos(ea.rows, min(row, g.M - 1));
+      crow = cache_row(ea.rows, min(row, g.M - 1), p);
+      rp = ea.rope + int64_t(p) * kDh;
+    }
     float hsq = 0.f;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      const int r = wv, l = lane;
-      float v = ((red[0][0][ct][r][l] + red[1][0][ct][r][l]) + red[2][0][ct][r][l]) + red[3][0][ct][r][l];
-      if constexpr (AM == 2) v = v / rrms[4 * (l >> 4) + r];
-      const int row = m0 + 4 * (l >> 4) + r, col = n0 + 16 * ct + (l & 15);
-      float* o = g.out + (EPI == kEpiStore ? int64_t(row) * g.ldo + col : act_index(row, col, g.N, 0));
-      if (row < g.M) {
-        if constexpr (EPI == kEpiStore) {
-          *o = v;
-        } else {
-          const float hv = hold[ct] + v;
-          *o = hv;
-          if constexpr (EPI == kEpiResidNorm) {
-            put_split(g.e.act + act_index(row, col, g.N, 0), g.e.act_plane, bf2f(g.e.xscale[col]) * hv);
-            hsq += hv * hv;
-          }
+    for (int i = 0; i < NI; ++i) {
+      const int ct = wv + NW * i;
+      if (ct >= ctn) break;
+      f32x4 v = rd[0][ct][lane];
+#pragma unroll
+      for (int w2 = 1; w2 < NW; ++w2) v += rd[w2][ct][lane];
+      if constexpr (AM == 2) v *= rrms[16 * rt + orow];
+      const int col = n0 + 16 * ct + ocol;
+      if (!live) continue;
+      if constexpr (EPI == kEpiStore) {
+        *reinterpret_cast<f32x4*>(g.out + int64_t(row) * g.ldo + col) = v;
+      } else if constexpr (kResid) {
+        v += hold[i];
+        const int64_t at = act_index(row, col, g.N, 0);
+        *reinterpret_cast<f32x4*>(g.out + at) = v;
+        if (ea.act) {
+          const uint2 sc = *reinterpret_cast<const uint2*>(ea.xscale + col);
+          const f32x4 x = {__uint_as_float(sc.x << 16) * v[0], __uint_as_float(sc.x & 0xffff0000u) * v[1],
+                           __uint_as_float(sc.y << 16) * v[2], __uint_as_float(sc.y & 0xffff0000u) * v[3]};
+          uint2 hi, lo;
+          split2(x[0], x[1], hi.x, lo.x);
+          split2(x[2], x[3], hi.y, lo.y);
+          *reinterpret_cast<uint2*>(ea.act + at) = hi;
+          *reinterpret_cast<uint2*>(ea.act + ea.act_plane + at) = lo;
+          hsq += ((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]) + v[3] * v[3];
         }
-      }
-    }
-    if constexpr (EPI == kEpiResidNorm) {   // the row's 16 CT columns: 16 lanes, in a fixed order
-      hsq = sum16_lanes(hsq);
-      const int row = m0 + 4 * (lane >> 4) + wv;
-      if ((lane & 15) == 0 && row < g.M) g.e.ssq[int64_t(row) * C + c] = hsq;
-    }
-  } else {
-    // one column pair (lanes l, l + 1 of a row) per thread
-    for (int idx = threadIdx.x; idx < RT * CT * 128; idx += 256) {
-      const int tc = idx >> 7, rt = tc / CT, ct = tc % CT, e = idx & 127, r = e >> 5,
-                l = 16 * ((e >> 3) & 3) + 2 * (e & 7);
-      float v0 = ((red[0][rt][ct][r][l] + red[1][rt][ct][r][l]) + red[2][rt][ct][r][l]) + red[3][rt][ct][r][l];
-      float v1 = ((red[0][rt][ct][r][l + 1] + red[1][rt][ct][r][l + 1]) + red[2][rt][ct][r][l + 1]) +
-                 red[3][rt][ct][r][l + 1];
-      if constexpr (AM == 2) {
-        v0 = v0 / rrms[16 * rt + 4 * (l >> 4) + r];
-        v1 = v1 / rrms[16 * rt + 4 * (l >> 4) + r];
-      }
-      const int row = m0 + 16 * rt + 4 * (l >> 4) + r, col = n0 + 16 * ct + (l & 15);
-      if (row >= g.M || ct >= ctn) continue;
-      const EpiArgs& ea = g.e;
-      if constexpr (EPI == kEpiSwiglu) {
+      } else if constexpr (EPI == kEpiSwiglu) {
         // (the tile copy orders the gate/up pairs by the down projection's input positions)
-        const int F = g.N / 2, f = col >> 1;
-        put_split(ea.act + act_index(row, f, F, 0), ea.act_plane, swiglu(v0, v1));
+        const int64_t at = act_index(row, col >> 1, g.N / 2, 0);
+        uint32_t hi, lo;
+        split2(swiglu(v[0], v[1]), swiglu(v[2], v[3]), hi, lo);
+        *reinterpret_cast<uint32_t*>(ea.act + at) = hi;
+        *reinterpret_cast<uint32_t*>(ea.act + ea.act_plane + at) = lo;
       } else {
-        const int p = row_pos(ea.rows, row);
-        const int64_t crow = cache_row(ea.rows, row, p);
-        const int head = col / kDh, ri = (col % kDh) >> 1;
-        const float c = ea.rope[int64_t(p) * kDh + ri], sg = ea.rope[int64_t(p) * kDh + kDh / 2 + ri];
-        const bool isv = head >= ea.H + ea.KV;
-        const int gi = isv ? head - ea.H - ea.KV : head - ea.H;
-        uint16_t* cp = (isv ? ea.vc : ea.kc) + (int64_t(gi) * ea.rows.pool + crow) * kDh;
-        qkv_pair(v0, v1, c, sg, col, ea.H, ea.KV, ea.qkv + int64_t(row) * g.N + head * kDh, cp);
+        qkv_quad(v, rp, col, ea.H, ea.KV, ea.qkv + int64_t(row) * g.N, ea.kc, ea.vc, int64_t(ea.rows.pool), crow);
       }
+    }
+    if constexpr (kResid) {   // the wave's columns of the row: four lanes, in a fixed order
+      hsq += __shfl_xor(hsq, 16);
+      hsq += __shfl_xor(hsq, 32);
+      if (lane < 16) hs[rt][wv][lane] = hsq;
+    }
+  }
+  if (kResid && g.e.act) {   // the waves' parts of each row's sum, in wave order
+    __syncthreads();
+    const int row = m0 + int(threadIdx.x);
+    if (threadIdx.x < 16 * RT && row < g.M) {
+      float sum = hs[threadIdx.x >> 4][0][threadIdx.x & 15];
+#pragma unroll
+      for (int w2 = 1; w2 < NW; ++w2) sum += hs[threadIdx.x >> 4][w2][threadIdx.x & 15];
+      g.e.ssq[int64_t(row) * C + c] = sum;
     }
   }
 }
@@ -1062,44 +1126,66 @@ static size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // Widest projection mx_gemm_rows takes with weights in row order: wider ones (the 306M gate/up,
 // 5632 outputs) run faster on the split-K kernel (measured: 128-token prefill 1.95 -> 1.79 ms).
-// With the weights in tile order it takes every width (gate/up at 128 rows: 18.7 -> 10.1 us).
 constexpr int kRowsMaxN = 4096;
 
-// Column tiles (of 16) per workgroup of mx_gemm_rows: the widest that still gives about one
-// workgroup per compute unit; 0 when the projection has too few output tiles for it (few rows),
-// or too short a K for every wave to take a step, and the split-K kernel runs instead.
-// With the weights in tile order (tw) every projection takes it (the fused epilogues and the
-// folded norms live there): the widest that gives about one workgroup per compute unit, else 1.
-// (Workgroups owning 2 or 4 row tiles, which read each weight tile for 32 or 64 rows, measured
-// slower: 128-token prefill 1.16 -> 1.36 / 1.70 ms.)
-static int rows_ct(int M, int N, int K, bool tw) {
+// Column tiles (of 16) per workgroup of mx_gemm_rows with weights in row order: the widest that still
+// gives about one workgroup per compute unit; 0 when the projection has too few output tiles for it
+// (few rows), or too short a K for every wave to take a step, and the split-K kernel runs instead.
+static int rows_ct(int M, int N, int K) {
   const int T = (M + 15) / 16, n16 = N / 16;
-  if (K / kBK < 4) return 0;
-  if (!tw && (M < 48 || N > kRowsMaxN)) return 0;
+  if (K / kBK < 4 || M < 48 || N > kRowsMaxN) return 0;
   for (int ct : {8, 6, 4, 3, 2, 1})
     if (n16 % ct == 0 && T * (n16 / ct) >= 224) return ct;
-  return tw ? 1 : 0;
+  return 0;
 }
 
-// Workgroups owning two row tiles (tile-order weights, pair epilogues): when one row tile per
-// workgroup needs more workgroups than compute units, the column tiles (6, 8 or 4, the last group
-// ragged) of a grid of 224-256 workgroups, else 0.  Every weight tile then serves 32 rows, and one
-// pass over the CUs does the whole projection (128-token gate/up, 352 column tiles: 13.3 -> 9.2 us
-// in a microbenchmark with weights that miss the last-level cache).
-static int rows_ct2(int M, int N, int K, bool tw) {
-  const int ct1 = rows_ct(M, N, K, tw), T = (M + 15) / 16, n16 = N / 16;
-  if (!tw || ct1 <= 0 || T < 2 || T * (n16 / ct1) <= 256) return 0;
-  for (int ct : {6, 8, 4}) {
-    const int wg = ((T + 1) / 2) * ((n16 + ct - 1) / ct);
-    if (wg >= 224 && wg <= 256) return ct;
+// Output tile of a workgroup of mx_gemm_rows with weights in tile order: RT x CT tiles of 16.
+struct RowsTile {
+  int rt, ct, nw;   // row tiles, column tiles, waves
+};
+constexpr RowsTile kRowsTiles[] = {{1, 1, 8}, {1, 1, 4}, {1, 2, 4}, {1, 3, 4}, {1, 4, 4}, {1, 6, 4}, {2, 2, 4},
+                                   {2, 3, 4}, {2, 4, 4}, {2, 6, 4}, {4, 3, 4}, {4, 4, 4}, {4, 6, 4}, {4, 11, 4}};
+
+// The tile of a projection, from a model of its time (us) fitted to cold-weight runs of the 306M
+// projections at 5..511 rows (within ~10 % of each; e.g. 511-row gate/up: 4 x 11 19.0 us, 2 x 6
+// 20.5, 4 x 6 25.2, 1 x 8 -- the old choice -- 27.4; 128-row gate/up 2 x 6 8.9, 1 x 3 11.2; 24-row
+// 1 x 3 5.7, 1 x 2 6.9): launch, first loads and drain 2.6; every K step moves 2 RT + CT operand
+// fragments into the CU (13 ns each); the epilogue takes 0.19 per tile; workgroups past one per
+// CU cost a share of both where two fit a CU's registers (up to 12 tiles), whole passes where not.
+// max_groups: an upper limit on column groups (0: none).
+static RowsTile rows_tile(int M, int N, int K, int max_groups = 0) {
+  const int T = (M + 15) / 16, n16 = N / 16, S = K / kBK;
+  RowsTile best = kRowsTiles[0];
+  double best_cost = 1e30;
+  for (const RowsTile& t : kRowsTiles) {
+    const int C = (n16 + t.ct - 1) / t.ct;
+    if (max_groups && C > max_groups) continue;
+    // one column of tiles: 8 waves where a wave of 4 would walk a long K or the CU is otherwise idle
+    if (t.rt * t.ct == 1 && (t.nw == 8) != (S >= 64 || T == 1)) continue;
+    const int wg = ((T + t.rt - 1) / t.rt) * C;
+    const double step = 0.013 * (2 * t.rt + t.ct) * S, epi = 0.19 * t.rt * t.ct;
+    const double cost = t.rt * t.ct <= 12 ? std::max(1.0, wg / 256.0) * step + epi + (wg > 256 ? 0.4 : 0.0)
+                                          : ((wg + 255) / 256) * (step + epi);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = t;
+    }
   }
-  return 0;
+  return best;
+}
+
+// Column groups of the O and down projections, which leave one partial sum of h^2 each per row (the
+// consumer takes up to 64).
+constexpr int kMaxGroups = 64;
+static int resid_groups(int M, int N, int K) {
+  const int ct = rows_tile(M, N, K, kMaxGroups).ct;
+  return (N / 16 + ct - 1) / ct;
 }
 
 // K splits of a projection: 1 for mx_gemm_rows, else enough split-K workgroups to occupy every
 // compute unit, at least 4 K steps each
 static int splits_for(int M, int N, int K, int bm, bool tw) {
-  if (rows_ct(M, N, K, tw) > 0) return 1;
+  if (tw || rows_ct(M, N, K) > 0) return 1;
   const int tiles = (N / kBN) * ((M + bm - 1) / bm);
   int s = 1;
   while (tiles * s < 256 && (K / kBK) / (2 * s) >= 4 && 2 * s <= kMaxSplitK) s *= 2;
@@ -1150,24 +1236,26 @@ static bool mx_config_ok(const msd_config* c) {
   return true;
 }
 
-template <int AM, bool TW, int EPI = kEpiStore>
-static void launch_rows(int ct, dim3 grid, hipStream_t s, const GemmArgs& g) {
+static void launch_rows_packed(int ct, int grid, hipStream_t s, const GemmArgs& g) {
   switch (ct) {
-    case 8: hipLaunchKernelGGL((mx_gemm_rows<8, 3, AM, TW, EPI>), grid, dim3(256), 0, s, g); break;
-    case 6: hipLaunchKernelGGL((mx_gemm_rows<6, 3, AM, TW, EPI>), grid, dim3(256), 0, s, g); break;
-    case 4: hipLaunchKernelGGL((mx_gemm_rows<4, 4, AM, TW, EPI>), grid, dim3(256), 0, s, g); break;
-    case 3: hipLaunchKernelGGL((mx_gemm_rows<3, 4, AM, TW, EPI>), grid, dim3(256), 0, s, g); break;
-    case 2: hipLaunchKernelGGL((mx_gemm_rows<2, 4, AM, TW, EPI>), grid, dim3(256), 0, s, g); break;
-    default: hipLaunchKernelGGL((mx_gemm_rows<1, 4, AM, TW, EPI>), grid, dim3(256), 0, s, g); break;
+    case 8: hipLaunchKernelGGL((mx_gemm_rows<1, 8, 3, 4, 1, false, kEpiStore>), dim3(grid), dim3(256), 0, s, g); break;
+    case 6: hipLaunchKernelGGL((mx_gemm_rows<1, 6, 3, 4, 1, false, kEpiStore>), dim3(grid), dim3(256), 0, s, g); break;
+    case 4: hipLaunchKernelGGL((mx_gemm_rows<1, 4, 4, 4, 1, false, kEpiStore>), dim3(grid), dim3(256), 0, s, g); break;
+    case 3: hipLaunchKernelGGL((mx_gemm_rows<1, 3, 4, 4, 1, false, kEpiStore>), dim3(grid), dim3(256), 0, s, g); break;
+    case 2: hipLaunchKernelGGL((mx_gemm_rows<1, 2, 4, 4, 1, false, kEpiStore>), dim3(grid), dim3(256), 0, s, g); break;
+    default: hipLaunchKernelGGL((mx_gemm_rows<1, 1, 4, 4, 1, false, kEpiStore>), dim3(grid), dim3(256), 0, s, g); break;
   }
 }
 
-template <int AM, int EPI>
-static void launch_rows2(int ct, dim3 grid, hipStream_t s, const GemmArgs& g) {
-  switch (ct) {
-    case 8: hipLaunchKernelGGL((mx_gemm_rows<8, 2, AM, true, EPI, 2>), grid, dim3(256), 0, s, g); break;
-    case 6: hipLaunchKernelGGL((mx_gemm_rows<6, 2, AM, true, EPI, 2>), grid, dim3(256), 0, s, g); break;
-    default: hipLaunchKernelGGL((mx_gemm_rows<4, 2, AM, true, EPI, 2>), grid, dim3(256), 0, s, g); break;
+// K steps in flight per wave: 4 while the tile leaves the registers for it
+template <int AM, int EPI, int I = 0>
+static void launch_rows_tiles(const RowsTile& t, int grid, hipStream_t s, const GemmArgs& g) {
+  constexpr RowsTile k = kRowsTiles[I];
+  if (t.rt == k.rt && t.ct == k.ct && t.nw == k.nw) {
+    constexpr int P = k.rt == 1 && k.ct <= 4 ? 4 : (k.rt * k.ct <= 6 ? 3 : 2);
+    hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI>), dim3(grid), dim3(64 * k.nw), 0, s, g);
+  } else if constexpr (I + 1 < int(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))) {
+    launch_rows_tiles<AM, EPI, I + 1>(t, grid, s, g);
   }
 }
 
@@ -1191,29 +1279,21 @@ static hipError_t gemm(const uint16_t* A, int64_t a_plane, int lda, const uint16
                        const EpiArgs* ea = nullptr, const float* ssq = nullptr, int nssq = 0) {
   GemmArgs g{A, a_plane, W, out, M, N, K, lda, ldo, splits, ea ? *ea : EpiArgs{}, ssq, nssq};
   const int am = ssq ? 2 : (lda == 0 ? 1 : 0);
-  const int ct = splits == 1 && rows_ok && am > 0 ? rows_ct(M, N, K, tw) : 0;
-  if ((epi != kEpiStore || am == 2) && !(ct > 0 && tw)) return hipErrorInvalidValue;
-  if ((epi == kEpiQkv || epi == kEpiSwiglu || epi == kEpiResidNorm) && !ea) return hipErrorInvalidValue;
-  if (am == 2 && (lda != 0 || nssq < 1 || nssq > 64)) return hipErrorInvalidValue;
-  if (epi == kEpiResidNorm && (!ea->act || !ea->xscale || !ea->ssq || N / (16 * ct) > 64)) return hipErrorInvalidValue;
-  const int ct2 = ct > 0 && (epi == kEpiSwiglu || epi == kEpiQkv) ? rows_ct2(M, N, K, tw) : 0;
-  if (ct2 > 0) {
-    const int TG = ((M + 15) / 16 + 1) / 2, C = (N / 16 + ct2 - 1) / ct2;
-    const dim3 grid(8 * ((C + 7) / 8) * TG);
-    if (am == 2 && epi == kEpiQkv) launch_rows2<2, kEpiQkv>(ct2, grid, s, g);
-    else if (am == 2 && epi == kEpiSwiglu) launch_rows2<2, kEpiSwiglu>(ct2, grid, s, g);
+  if ((epi != kEpiStore) != tw || (epi != kEpiStore && (!ea || am == 0 || splits != 1)))
+    return hipErrorInvalidValue;
+  if (am == 2 && (lda != 0 || nssq < 1 || nssq > kMaxGroups || !tw)) return hipErrorInvalidValue;
+  const int T = (M + 15) / 16;
+  if (tw) {
+    const RowsTile t = rows_tile(M, N, K, epi == kEpiResid ? kMaxGroups : 0);
+    const int grid = ((T + t.rt - 1) / t.rt) * ((N / 16 + t.ct - 1) / t.ct);
+    if (am == 2 && epi == kEpiQkv) launch_rows_tiles<2, kEpiQkv>(t, grid, s, g);
+    else if (am == 2 && epi == kEpiSwiglu) launch_rows_tiles<2, kEpiSwiglu>(t, grid, s, g);
+    else if (am == 1 && epi == kEpiResid) launch_rows_tiles<1, kEpiResid>(t, grid, s, g);
     else return hipErrorInvalidValue;
     return hipGetLastError();
   }
-  if (ct > 0) {
-    const int T = (M + 15) / 16, C = N / (16 * ct);
-    const dim3 grid(8 * ((C + 7) / 8) * T);
-    if (am == 2 && epi == kEpiQkv) launch_rows<2, true, kEpiQkv>(ct, grid, s, g);
-    else if (am == 2 && epi == kEpiSwiglu) launch_rows<2, true, kEpiSwiglu>(ct, grid, s, g);
-    else if (am == 1 && tw && epi == kEpiResid) launch_rows<1, true, kEpiResid>(ct, grid, s, g);
-    else if (am == 1 && tw && epi == kEpiResidNorm) launch_rows<1, true, kEpiResidNorm>(ct, grid, s, g);
-    else if (am == 1 && !tw && epi == kEpiStore) launch_rows<1, false>(ct, grid, s, g);
-    else return hipErrorInvalidValue;
+  if (const int ct = splits == 1 && rows_ok && am == 1 ? rows_ct(M, N, K) : 0; ct > 0) {
+    launch_rows_packed(ct, T * (N / (16 * ct)), s, g);
     return hipGetLastError();
   }
   const int bm = bm_for(M);
@@ -1271,7 +1351,7 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
                 toff_sc = toff_dn + int64_t(d) * ff;
   // partial sums of h^2 per row that the O and down epilogues leave (one per column group); the
   // first layer's come from mx_embed (one per row)
-  const int cg_o = tw ? d / (16 * rows_ct(M, d, d, true)) : 0, cg_d = tw ? d / (16 * rows_ct(M, d, ff, true)) : 0;
+  const int cg_o = tw ? resid_groups(M, d, d) : 0, cg_d = tw ? resid_groups(M, d, ff) : 0;
   int pending = 0;
   err = hipSuccess;
   for (int l = 0; l < cfg->n_layers && err == hipSuccess; ++l) {
@@ -1308,7 +1388,7 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
       en.act_plane = pd;
       en.ssq = ssq;
       en.xscale = Tl + toff_sc + d;
-      if ((err = gemm(att, pd, 0, Tl + toff_o, true, M, d, d, h, d, 1, s, true, kEpiResidNorm, &en)) != hipSuccess)
+      if ((err = gemm(att, pd, 0, Tl + toff_o, true, M, d, d, h, d, 1, s, true, kEpiResid, &en)) != hipSuccess)
         break;
       EpiArgs eg{};
       eg.act = act;
@@ -1316,9 +1396,9 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
       if ((err = gemm(xn, pd, 0, Tl + toff_gu, true, M, 2 * ff, d, nullptr, 0, 1, s, true, kEpiSwiglu, &eg, ssq, cg_o)) !=
           hipSuccess)
         break;
-      if (!last) en.xscale = Tl + tile_layer_elems(cfg) + toff_sc;   // the next layer's RMSNorm1
-      if ((err = gemm(act, pf, 0, Tl + toff_dn, true, M, d, ff, h, d, 1, s, true, last ? kEpiResid : kEpiResidNorm,
-                      last ? nullptr : &en)) != hipSuccess)
+      if (last) en.act = nullptr;   // (the final norm reads h)
+      else en.xscale = Tl + tile_layer_elems(cfg) + toff_sc;   // the next layer's RMSNorm1
+      if ((err = gemm(act, pf, 0, Tl + toff_dn, true, M, d, ff, h, d, 1, s, true, kEpiResid, &en)) != hipSuccess)
         break;
       continue;
     }
