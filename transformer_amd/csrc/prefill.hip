@@ -192,17 +192,23 @@ struct GemmArgs {
 
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 u) { return __builtin_bit_cast(bf16x8, u); }
 
+// Two f32 values as hi/lo parts, packed (a in the low halves; v_cvt_pk_bf16_f32 rounds to nearest even).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  hi = pack2(a, b);
+  lo = pack2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
+}
+
 // Eight f32 values as hi/lo bf16 parts (hi = bf16(x), lo = bf16(x - hi)), packed as MFMA operands.
 __device__ __forceinline__ void split8(const float (&x)[8], uint4& hi, uint4& lo) {
-  uint32_t h[4], l[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint16_t h0 = f2bf(x[2 * i]), h1 = f2bf(x[2 * i + 1]);
-    h[i] = uint32_t(h0) | (uint32_t(h1) << 16);
-    l[i] = uint32_t(f2bf(x[2 * i] - bf2f(h0))) | (uint32_t(f2bf(x[2 * i + 1] - bf2f(h1))) << 16);
-  }
-  hi = make_uint4(h[0], h[1], h[2], h[3]);
-  lo = make_uint4(l[0], l[1], l[2], l[3]);
+  split2(x[0], x[1], hi.x, lo.x);
+  split2(x[2], x[3], hi.y, lo.y);
+  split2(x[4], x[5], hi.z, lo.z);
+  split2(x[6], x[7], hi.w, lo.w);
 }
 
 // f32 operands as hi/lo parts on the matrix cores: a b ~ ah bh + ah bl + al bh (the lo lo term,
@@ -315,17 +321,6 @@ __device__ __forceinline__ void qkv_pair(float s0, float s1, float c, float sg, 
     cp[d0] = f2bf(o0);
     cp[d1] = f2bf(o1);
   }
-}
-
-// Two f32 values as hi/lo parts, packed (a in the low halves; v_cvt_pk_bf16_f32 rounds to nearest even).
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
-}
-__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-  hi = pack2(a, b);
-  lo = pack2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
 }
 
 // Four outputs of the packed q/k/v rows col .. col + 3 (col a multiple of 4): qkv_pair for both pairs
@@ -763,12 +758,13 @@ __device__ __forceinline__ float row16_sum(float v) {
 // D: rows 4 (l / 16) + r of column l % 16.
 // The head outputs go to the O projection's input planes at their packed positions, or with
 // natural at their element index (the tile copy's O columns are in natural order).
-__global__ __launch_bounds__(256) void mx_attention_prefill(const float* qkv, int M, int H, int KV, uint16_t* att,
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv, int M, int H, int KV, uint16_t* att,
                                                             int64_t plane, int ldx, int natural) {
   constexpr int PS = 36;   // row stride (floats) of a wave's P tile in LDS: 16-byte reads of 16 rows spread over banks
-  __shared__ __align__(16) float sp[4][16 * PS];
-  __shared__ float sm[4][16], sl[4][16];
-  __shared__ float so[4][16][kDh + 4];
+  __shared__ __align__(16) float sp[NW][16 * PS];
+  __shared__ float sm[NW][16], sl[NW][16];
+  __shared__ float so[NW][16][kDh + 4];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
   const int h = blockIdx.x, g = h / (H / KV);
@@ -796,7 +792,7 @@ __global__ __launch_bounds__(256) void mx_attention_prefill(const float* qkv, in
     o[r] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   float* P = sp[wv];
-  for (int c = wv; c < nch; c += 4) {
+  for (int c = wv; c < nch; c += NW) {
     const int kb = 32 * c;
     // K rows (B of S: key kb + 16 t + r16, dims 32 ks + 8 kq ..) and V values (B of P V: keys
     // kb + 8 kq + e, dim 16 dt + r16), all requested before the first MFMA; keys past M read
@@ -875,13 +871,14 @@ __global__ __launch_bounds__(256) void mx_attention_prefill(const float* qkv, in
 #pragma unroll
     for (int r = 0; r < 4; ++r) so[wv][4 * kq + r][16 * dt + r16] = o[dt][r];
   __syncthreads();
+  if (threadIdx.x >= 256) return;
   const int qi = threadIdx.x >> 4, d4 = 4 * (threadIdx.x & 15);
   float mx = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) mx = fmaxf(mx, sm[w][qi]);
+  for (int w = 0; w < NW; ++w) mx = fmaxf(mx, sm[w][qi]);
   float L = 0.f, O[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < NW; ++w) {
     const float wt = sm[w][qi] == -INFINITY ? 0.f : expf(sm[w][qi] - mx);
     L += sl[w][qi] * wt;
 #pragma unroll
@@ -896,121 +893,211 @@ __global__ __launch_bounds__(256) void mx_attention_prefill(const float* qkv, in
     }
 }
 
-// Batched decode: row m (one sequence at position p = pos(m)) and head blockIdx.y attend over
-// the cached rows 0..p-1 of the sequence (bf16, through its page table) and the row's
-// current, un-rounded K/V (multi_sm_decode.py:182-221).  Wave w takes positions
-// [64w, 64w + 64) (contexts up to 512): each lane looks its position's cache row up, then the
-// wave requests its K rows (lane = position) and all its V values (lane = dimension) at once,
-// so the block costs two memory round trips; each wave keeps its own maximum and sum and the
-// waves' states are merged in LDS at the end.
+static void launch_attention_prefill(int M, int H, int KV, hipStream_t s, const float* qkv, uint16_t* att,
+                                     int64_t plane, int natural) {
+  const dim3 grid(H, (M + 15) / 16);
+  if (M > 128)
+    hipLaunchKernelGGL(mx_attention_prefill<8>, grid, dim3(512), 0, s, qkv, M, H, KV, att, plane, 0, natural);
+  else
+    hipLaunchKernelGGL(mx_attention_prefill<4>, grid, dim3(256), 0, s, qkv, M, H, KV, att, plane, 0, natural);
+}
+
+// Batched decode: row m = blockIdx.x (one sequence at position p = pos(m)) and the GH query heads
+// GH blockIdx.y .. (of one K/V head) attend over the cached rows 0..p-1 of the sequence (bf16, through
+// its page table) and the row's current, un-rounded K/V (multi_sm_decode.py:182-221).  What bounds it
+// is latency and load instructions, not bytes (24 rows of up to 384 positions: 21 MB when every head
+// reads its K/V): wave w takes the 32-position blocks w, w + 8, ..., the next block's rows requested
+// before the current one's arithmetic.  Lane l reads dims 8 (l % 8) .. + 8 of position 8 i + l / 8, i = 0..3,
+// of K and of V: whole rows, 1 KB per instruction (a lane per position for K and per dim for V took
+// 72 instructions per 64 positions and 64 cache lines per K instruction: 13.9 us for the 24 rows).  The
+// 8 lanes of a position add their partial scores with DPP, so every lane ends up with the weights of
+// exactly the V rows it holds; only (max, sum, output) partials go through LDS at the end.
 constexpr int kAttnWaves = 8;
-// Positions mx_attention_decode covers: wave w takes the 64-position blocks w, w + 8, ...
+// Positions mx_attention_decode covers.
 constexpr int kAttnMaxCtx = 2048;
+__device__ __forceinline__ float sum8_lanes(float v) {   // over each 8 consecutive lanes, as sum16_lanes
+  v += dpp<0xB1, 0xf>(v, 0.f);
+  v += dpp<0x4E, 0xf>(v, 0.f);
+  return v + dpp<0x141, 0xf>(v, 0.f);
+}
+template <int GH>
 __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const float* qkv, Rows rows, int H, int KV,
                                                                        const uint16_t* kc, const uint16_t* vc,
                                                                        uint16_t* att, int64_t plane, int ldx,
                                                                        int natural) {
-  __shared__ float sq[kDh], skc[kDh], svc[kDh];   // q, and the current position's f32 k and v
-  __shared__ float sp[kAttnWaves][64];
-  __shared__ int srow[kAttnWaves][64];
-  __shared__ float so[kAttnWaves][kDh];
-  __shared__ float sml[kAttnWaves][2];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int m = blockIdx.x, h = blockIdx.y, g = h / (H / KV);
+  // per wave and row of 16 lanes: the output's partial sums and the softmax denominator's
+  __shared__ float so[kAttnWaves][4][GH][kDh];
+  __shared__ float sl[kAttnWaves][4][GH];
+  __shared__ float sm[kAttnWaves][GH];
+  constexpr int kPos = 32, kLd = kPos / 8;   // positions per block, loads of K and of V per lane
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = lane >> 3, d8 = 8 * (lane & 7);
+  const int m = blockIdx.x, h0 = GH * blockIdx.y, g = h0 / (H / KV);
   const int nqkv = (H + 2 * KV) * kDh, d = H * kDh;
-  // q, the page-table entries of the first block and p are loaded together: the page-table load
-  // does not wait for p (every entry of a row is a sanitized page; p only selects which rows are
-  // cached positions), and no load sits under a branch (it would be waited for at the join)
   const float* qr = qkv + int64_t(m) * nqkv;
-  const int qsel = min(int(threadIdx.x) / kDh, 2);   // threads 0..63: q, 64..127: k, others: v
-  const float qv = qr[(qsel == 0 ? h : (qsel == 1 ? H + g : H + KV + g)) * kDh + (threadIdx.x & (kDh - 1))];
-  auto row_of = [&](int j) { return cache_row(rows, m, rows.pages ? min(j, rows.max_pages * kPage - 1) : j); };
-  int64_t cr = row_of(64 * wv + lane);
+  // the page-table loads do not wait for p (every entry of a row is a sanitized page; p only selects
+  // which rows are cached positions); positions past the table or past p read the row of position 0
+  auto page_of = [&](int page) {   // wave-uniform
+    return rows.pages ? rows.pages[int64_t(rows.batched ? m : 0) * rows.max_pages + min(page, rows.max_pages - 1)] : page;
+  };
+  int pg0 = page_of(2 * wv), pg1 = page_of(2 * wv + 1);
+  const int first = page_of(0);
   const int p = row_pos(rows, m);
-  if (threadIdx.x < 3 * kDh) (qsel == 0 ? sq : (qsel == 1 ? skc : svc))[threadIdx.x & (kDh - 1)] = qv;
-  const uint16_t* kg = kc + int64_t(g) * rows.pool * kDh;
-  const uint16_t* vg = vc + int64_t(g) * rows.pool * kDh;
-  __syncthreads();
-  float mx = -INFINITY, ls = 0.f, o = 0.f;
-  // blocks wv, wv + 8, ... up to the one holding p (each holds at least one position <= p);
-  // the first is taken as it is, later ones merged by log-sum-exp
-  for (int blk = wv; 64 * blk <= p; blk += kAttnWaves) {
-    const int j0 = 64 * blk, j = j0 + lane;
-    if (blk != wv) cr = row_of(j);
-    srow[wv][lane] = j < p ? int(cr) : 0;
-    __builtin_amdgcn_wave_barrier();
-    uint4 ku[kDh / 8];
-    const uint4* kr = reinterpret_cast<const uint4*>(kg + int64_t(srow[wv][lane]) * kDh);
+  float q[GH][8], kcur[8], vcur[8];
+  auto load8 = [&](const float* src, float (&x)[8]) {
+    const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
+    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+    x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+  };
 #pragma unroll
-    for (int e8 = 0; e8 < kDh / 8; ++e8) ku[e8] = kr[e8];
-    uint16_t vv[64];
+  for (int h = 0; h < GH; ++h) load8(qr + (h0 + h) * kDh + d8, q[h]);
+  load8(qr + (H + g) * kDh + d8, kcur);
+  load8(qr + (H + KV + g) * kDh + d8, vcur);
+  const uint16_t* kg = kc + int64_t(g) * rows.pool * kDh + d8;
+  const uint16_t* vg = vc + int64_t(g) * rows.pool * kDh + d8;
+  uint4 kb[2][kLd], vb[2][kLd];
+  auto load = [&](uint4 (&k)[kLd], uint4 (&v)[kLd], int blk, int p0, int p1) {
 #pragma unroll
-    for (int jj = 0; jj < 64; ++jj) vv[jj] = vg[int64_t(srow[wv][jj]) * kDh + lane];
-    float s = -INFINITY;
-    if (j < p) {
-      float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-      for (int e8 = 0; e8 < kDh / 8; ++e8) {
-        const uint32_t wds[4] = {ku[e8].x, ku[e8].y, ku[e8].z, ku[e8].w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          a0 += sq[8 * e8 + 2 * q] * __uint_as_float(wds[q] << 16);
-          a1 += sq[8 * e8 + 2 * q + 1] * __uint_as_float(wds[q] & 0xffff0000u);
-        }
-      }
-      s = (a0 + a1) * 0.125f;
-    } else if (j == p) {   // current position: f32 K from this row's projection
-      float a0 = 0.f, a1 = 0.f;
-      for (int e = 0; e < kDh; e += 2) {
-        a0 += sq[e] * skc[e];
-        a1 += sq[e + 1] * skc[e + 1];
-      }
-      s = (a0 + a1) * 0.125f;
+    for (int i = 0; i < kLd; ++i) {
+      const bool in = kPos * blk + 8 * i + sub < p;
+      const int64_t r = in ? int64_t(i < 2 ? p0 : p1) * kPage + (8 * i + sub) % kPage : int64_t(first) * kPage;
+      k[i] = *reinterpret_cast<const uint4*>(kg + r * kDh);
+      v[i] = *reinterpret_cast<const uint4*>(vg + r * kDh);
     }
-    const float bmx = wave_max(s);
-    const float e = (s == -INFINITY) ? 0.f : expf(s - bmx);
-    const float bls = wave_sum(e);
-    sp[wv][lane] = e;
-    __builtin_amdgcn_wave_barrier();
-    const float vcur = svc[lane];
-    float o4[4] = {0.f, 0.f, 0.f, 0.f};
+  };
+  const int nb = (p + kPos - 1) / kPos;
+  load(kb[0], vb[0], wv, pg0, pg1);
+  // the last wave starts from the current position (its first 8 lanes), the others from nothing
+  float mx[GH], ls[GH], o[GH][8];
 #pragma unroll
-    for (int jj = 0; jj < 64; ++jj) {
-      const float v = j0 + jj < p ? bf2f(vv[jj]) : (j0 + jj == p ? vcur : 0.f);
-      o4[jj & 3] += sp[wv][jj] * v;
-    }
-    const float bo = (o4[0] + o4[1]) + (o4[2] + o4[3]);
-    if (blk == wv) {
-      mx = bmx;
-      ls = bls;
-      o = bo;
-    } else {
-      const float M = fmaxf(mx, bmx);
-      const float a0 = expf(mx - M), a1 = expf(bmx - M);
-      ls = ls * a0 + bls * a1;
-      o = o * a0 + bo * a1;
-      mx = M;
-    }
-    __builtin_amdgcn_wave_barrier();   // srow and sp are rewritten by the next block
+  for (int h = 0; h < GH; ++h) {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += q[h][e] * kcur[e];
+    s = sum8_lanes(s) * 0.125f;
+    const bool cur = wv == kAttnWaves - 1;
+    mx[h] = cur ? s : -INFINITY;
+    ls[h] = cur && sub == 0 ? 1.f : 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[h][e] = cur && sub == 0 ? vcur[e] : 0.f;
   }
-  so[wv][lane] = o;
-  if (lane == 0) {
-    sml[wv][0] = mx;
-    sml[wv][1] = ls;
+  auto unpack = [](uint4 u, float (&x)[8]) {
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[2 * e] = __uint_as_float(w[e] << 16);
+      x[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+    }
+  };
+  auto block = [&](const uint4 (&k)[kLd], const uint4 (&v)[kLd], int blk) {
+    float s[GH][kLd], old[GH];
+#pragma unroll
+    for (int h = 0; h < GH; ++h) old[h] = mx[h];
+#pragma unroll
+    for (int i = 0; i < kLd; ++i) {
+      float x[8];
+      unpack(k[i], x);
+      const bool in = kPos * blk + 8 * i + sub < p;
+#pragma unroll
+      for (int h = 0; h < GH; ++h) {
+        float a = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a += q[h][e] * x[e];
+        s[h][i] = in ? sum8_lanes(a) * 0.125f : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < GH; ++h) {
+      const float bm = wave_max(fmaxf(fmaxf(s[h][0], s[h][1]), fmaxf(s[h][2], s[h][3])));
+      mx[h] = fmaxf(mx[h], bm);
+      const float nm = mx[h] == -INFINITY ? 0.f : mx[h];   // (only scores of -inf so far: weights 0)
+      const float al = expf(old[h] - nm);
+#pragma unroll
+      for (int i = 0; i < kLd; ++i) s[h][i] = expf(s[h][i] - nm);
+      ls[h] = ls[h] * al + ((s[h][0] + s[h][1]) + (s[h][2] + s[h][3]));
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[h][e] *= al;
+    }
+#pragma unroll
+    for (int i = 0; i < kLd; ++i) {
+      float x[8];
+      unpack(v[i], x);
+#pragma unroll
+      for (int h = 0; h < GH; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[h][e] += s[h][i] * x[e];
+    }
+  };
+  for (int blk = wv; blk < nb; blk += 2 * kAttnWaves) {
+    const int b1 = blk + kAttnWaves, b2 = b1 + kAttnWaves;
+    if (b1 < nb) load(kb[1], vb[1], b1, page_of(2 * b1), page_of(2 * b1 + 1));
+    block(kb[0], vb[0], blk);
+    if (b2 < nb) load(kb[0], vb[0], b2, page_of(2 * b2), page_of(2 * b2 + 1));
+    if (b1 < nb) block(kb[1], vb[1], b1);
+  }
+  // the two positions of each row of 16 lanes are added here, the rest by the merge below
+#pragma unroll
+  for (int h = 0; h < GH; ++h) {
+    const float l2 = ls[h] + dpp<0x128, 0xf>(ls[h], 0.f);   // row_ror 8: lane ^ 8
+    if ((lane & 15) == 0) sl[wv][lane >> 4][h] = l2;
+    if (lane == 0) sm[wv][h] = mx[h];
+    float r[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = o[h][e] + dpp<0x128, 0xf>(o[h][e], 0.f);
+    if ((lane & 8) == 0) {
+      float* dst = so[wv][lane >> 4][h] + d8;
+      *reinterpret_cast<float4*>(dst) = make_float4(r[0], r[1], r[2], r[3]);
+      *reinterpret_cast<float4*>(dst + 4) = make_float4(r[4], r[5], r[6], r[7]);
+    }
   }
   __syncthreads();
-  if (wv == 0) {
+  // dims 2 t, 2 t + 1 of a head: the waves' states merged by log-sum-exp (waves without a position
+  // carry weight 0)
+  if (threadIdx.x < GH * kDh / 2) {
+    const int h = threadIdx.x / (kDh / 2), e = 2 * (threadIdx.x % (kDh / 2));
     float M = -INFINITY;
-    for (int w = 0; w < kAttnWaves; ++w) M = fmaxf(M, sml[w][0]);
-    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) M = fmaxf(M, sm[w][h]);
+    float num0 = 0.f, num1 = 0.f, den = 0.f;
+#pragma unroll
     for (int w = 0; w < kAttnWaves; ++w) {
-      if (sml[w][0] == -INFINITY) continue;
-      const float a = expf(sml[w][0] - M);
-      num += a * so[w][lane];
-      den += a * sml[w][1];
+      const float a = expf(sm[w][h] - M);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float2 v = *reinterpret_cast<const float2*>(so[w][r][h] + e);
+        num0 += a * v.x;
+        num1 += a * v.y;
+        den += a * sl[w][r][h];
+      }
     }
-    put_split(att + act_index(m, natural ? h * kDh + lane : perm_pos(h * kDh + lane, d), d, ldx), plane, num / den);
+    num0 /= den;
+    num1 /= den;
+    const int el = (h0 + h) * kDh + e;
+    if (natural) {
+      uint32_t hi, lo;
+      split2(num0, num1, hi, lo);
+      const int64_t at = act_index(m, el, d, ldx);
+      *reinterpret_cast<uint32_t*>(att + at) = hi;
+      *reinterpret_cast<uint32_t*>(att + plane + at) = lo;
+    } else {
+      put_split(att + act_index(m, perm_pos(el, d), d, ldx), plane, num0);
+      put_split(att + act_index(m, perm_pos(el + 1, d), d, ldx), plane, num1);
+    }
   }
+}
+
+// Heads per workgroup: as many of a K/V head's as leave about a workgroup per CU (each reads the K/V
+// rows once for its heads; fewer workgroups than CUs cost more than the shared reads save).
+static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const float* qkv, const Rows& rows,
+                                    const uint16_t* kc, const uint16_t* vc, uint16_t* att, int64_t plane,
+                                    int natural) {
+  const int G = H / KV;
+  auto go = [&](auto k, int gh) {
+    hipLaunchKernelGGL(k, dim3(M, H / gh), dim3(64 * kAttnWaves), 0, s, qkv, rows, H, KV, kc, vc, att, plane, 0, natural);
+  };
+  if (G % 4 == 0 && M * H / 4 >= 160) go(mx_attention_decode<4>, 4);
+  else if (G % 2 == 0 && M * H / 2 >= 160) go(mx_attention_decode<2>, 2);
+  else go(mx_attention_decode<1>, 1);
 }
 
 // argmax of each row of logits (lowest index on ties): out[2*row] = index, out[2*row+1] = status
@@ -1379,10 +1466,9 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
           hipSuccess)
         break;
       if (prefill)
-        hipLaunchKernelGGL(mx_attention_prefill, dim3(H, (M + 15) / 16), dim3(256), 0, s, qkv, M, H, KV, att, pd, 0, 1);
+        launch_attention_prefill(M, H, KV, s, qkv, att, pd, 1);
       else
-        hipLaunchKernelGGL(mx_attention_decode, dim3(M, H), dim3(64 * kAttnWaves), 0, s, qkv, rows, H, KV, kc, vc,
-                           att, pd, 0, 1);
+        launch_attention_decode(M, H, KV, s, qkv, rows, kc, vc, att, pd, 1);
       EpiArgs en{};   // the next RMSNorm's input planes and partial sums of h^2
       en.act = xn;
       en.act_plane = pd;
@@ -1407,10 +1493,9 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
     hipLaunchKernelGGL(mx_qkv_fin, dim3(M, (nqkv / 4 + 255) / 256), dim3(256), 0, s, part, sq, M, H, KV, wt.rope, rows,
                        kc, vc, qkv);
     if (prefill)
-      hipLaunchKernelGGL(mx_attention_prefill, dim3(H, (M + 15) / 16), dim3(256), 0, s, qkv, M, H, KV, att, pd, 0, 0);
+      launch_attention_prefill(M, H, KV, s, qkv, att, pd, 0);
     else
-      hipLaunchKernelGGL(mx_attention_decode, dim3(M, H), dim3(64 * kAttnWaves), 0, s, qkv, rows, H, KV, kc, vc, att,
-                         pd, 0, 0);
+      launch_attention_decode(M, H, KV, s, qkv, rows, kc, vc, att, pd, 0);
     if ((err = gemm(att, pd, 0, Wl + off_o, false, M, d, d, part, d, so, s)) != hipSuccess) break;
     hipLaunchKernelGGL(mx_norm, dim3(M), dim3(kNormThreads), 0, s, h, part, so, M, d, Wl + off_ln2, xn, pd, 0, 0, 0);
     if ((err = gemm(xn, pd, 0, Wl + off_gu, false, M, 2 * ff, d, part, 2 * ff, sg, s)) != hipSuccess) break;
