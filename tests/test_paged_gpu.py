@@ -167,6 +167,36 @@ def test_batched_step_matches_single_sequence_rows():
         assert n1[0] == nxt[b]
 
 
+def test_batch_of_64_matches_batches_of_16():
+    """Four heads per attention workgroup (64 rows) against one (16 rows), and their projection
+    tiles: the same sums but for the f32 order of a projection's K steps."""
+    cfg = dict(vocab_size=512, d_model=1024, n_heads=16, n_kv_heads=4, n_layers=2, d_head=64, d_ff=2816,
+               context_len=512)
+    w = prepare_decode_weights_nlayer(make_params(cfg, seed=4), cfg)
+    rng = np.random.default_rng(5)
+    B, per = 64, 512 // PAGE
+    pos = rng.integers(0, 512, B)
+    pos[:6] = [0, 1, 31, 32, 257, 511]
+    table = rng.permutation(B * per).reshape(B, per)
+    toks = torch.from_numpy(rng.integers(0, 512, B).astype(np.int32)).cuda()
+    data = torch.randn(PagePool(cfg, B * per).data.shape, device="cuda").to(torch.bfloat16)
+
+    def run(rows):
+        pool = PagePool(cfg, B * per)
+        pool.data.copy_(data)
+        bd = PagedBatchDecoder(w, cfg, pool, len(rows))
+        for i, b in enumerate(rows):
+            bd.set_pages(i, [int(x) for x in table[b]])
+        out = bd.launch(toks[rows].contiguous(), torch.from_numpy(pos[rows].astype(np.int32)).cuda())
+        torch.cuda.synchronize()
+        assert not out.reshape(-1, 2)[:, 1].any()
+        return bd.logits.float().cpu().numpy()
+
+    whole = run(list(range(B)))
+    parts = np.concatenate([run(list(range(b, b + 16))) for b in range(0, B, 16)])
+    assert np.linalg.norm(whole - parts) <= 1e-4 * np.linalg.norm(parts)
+
+
 def test_bad_positions_and_pages_are_reported():
     params = make_params(TINY, seed=0)
     bd, pool, tables, prompts, first = _setup(TINY, params, 2, [16, 16], 4, 32, seed=7)

@@ -109,6 +109,30 @@ def test_pack_tiles_layout(tiny):
     assert got.shape == want.shape and np.array_equal(got, want)
 
 
+WIDE = dict(vocab_size=512, d_model=1024, n_heads=16, n_kv_heads=4, n_layers=2, d_head=64, d_ff=2816,
+            context_len=1024)
+
+
+@pytest.fixture(scope="module")
+def wide():
+    return prepare_decode_weights_nlayer(make_params(WIDE, seed=3), WIDE)
+
+
+@pytest.mark.parametrize("T", [15, 17, 48, 65, 129, 255, 300, 511, 1000])
+def test_tile_choices_match_the_packed_rows(wide, T):
+    """The output tiles (1-4 row tiles x 1-11 column tiles, short last groups and row tiles) and the
+    attention's waves and key padding, against the packed-row path.  Both carry every projection
+    input to 2^-17 (7.6e-6) and sum in f32; nine projections in a chain stay within 1e-4."""
+    toks = make_prompt(T, WIDE["vocab_size"], seed=T)
+    la, _, out, kv = _run(wide, WIDE, toks)
+    lb, _, out2, kv2 = _run(wide, WIDE, toks, tiles=False)
+    assert out[1] == 0 and out2[1] == 0
+    assert np.linalg.norm(la - lb) <= 1e-4 * np.linalg.norm(lb)
+    a, b = kv.float(), kv2.float()
+    assert float((a - b).abs().max()) <= 2 ** -7 * float(b.abs().max())   # at most a bf16 step
+    assert float((a - b).norm()) <= 1e-3 * float(b.norm())
+
+
 def test_306m_prefill_128_matches_oracle(m306):
     """The prefill of a 128-token prompt on the 306M configuration."""
     params, w = m306

@@ -24,7 +24,8 @@
 //   mx_norm        residual += split-K partials of the previous projection (in split order),
 //                  then RMSNorm -> bf16 activations in the weights' permuted input order
 //   mx_gemm        q/k/v projection, split-K partials
-//   mx_qkv_fin     sum of the partials, RoPE on q/k, f32 q/k/v, bf16 K/V cache rows
+//   mx_qkv_fin     sum of the partials, RoPE on q/k, f32 q/k/v (a prefill: K and V as operand planes),
+//                  bf16 K/V cache rows
 //   attention      prefill: causal GQA over the prompt; batched decode: each sequence over
 //                  its cached rows plus its current K/V
 //   mx_gemm        O projection, split-K partials
@@ -177,7 +178,20 @@ struct EpiArgs {
   uint16_t* vc;
   float* qkv;
   int H, KV;
+  uint16_t* kvp;   // QKV of a prefill: the attention's K/V operand planes (below), else NULL
+  int MP;
 };
+
+// A prefill's K and V for its own attention, as bf16 hi/lo planes [K hi | K lo | V hi | V lo] of KV * MP *
+// 64 values (MP: rows padded to 32), each K/V head in the tile order of the matrix-core operand
+// that reads it: K as rows of 64 dims (16 keys x 32 dims per tile), V as the transpose (16 dims x 32
+// keys per tile).
+__device__ __forceinline__ int64_t k_plane_index(int g, int key, int dim, int MP) {
+  return int64_t(g) * MP * kDh + act_index(key, dim, kDh, 0);
+}
+__device__ __forceinline__ int64_t v_plane_index(int g, int key, int dim, int MP) {
+  return int64_t(g) * MP * kDh + act_index(dim, key, MP, 0);
+}
 
 struct GemmArgs {
   const uint16_t* A;   // [M][lda] bf16 (or tile order, see act_index): the hi parts; the lo
@@ -302,36 +316,40 @@ __global__ __launch_bounds__(256) void mx_gemm(GemmArgs g) {
       }
 }
 
-// SwiGLU of a gate/up pair (packed rows 2f, 2f + 1; model.py:159).
-__device__ __forceinline__ float swiglu(float g, float u) { return (g * (1.f / (1.f + expf(-g)))) * u; }
+// exp(x) by the hardware base-2 exponential (x log2(e) rounded once: |x| 2^-24 relative)
+__device__ __forceinline__ float exp_hw(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
-// Outputs s0, s1 of the packed q/k/v rows col, col + 1 (col even) of row m, whose position has
-// RoPE factors c, sg for this pair: q and k pairs are rotated (dims i, i + 32; model.py:110-117),
-// v is stored as projected; f32 q/k/v in natural head-dim order to `q`, bf16 K/V to the cache
-// row cp (multi_sm_decode.py:179-180).
-__device__ __forceinline__ void qkv_pair(float s0, float s1, float c, float sg, int col, int H, int KV, float* q,
-                                         uint16_t* cp) {
-  const int head = col / kDh, rr = col % kDh, ri = rr >> 1;
-  const bool rot = head < H + KV;
-  const float o0 = rot ? s0 * c - s1 * sg : s0, o1 = rot ? s0 * sg + s1 * c : s1;
-  const int d0 = rot ? ri : rr, d1 = rot ? ri + kDh / 2 : rr + 1;
-  q[d0] = o0;
-  q[d1] = o1;
-  if (head >= H) {
-    cp[d0] = f2bf(o0);
-    cp[d1] = f2bf(o1);
-  }
+// SwiGLU of a gate/up pair (packed rows 2f, 2f + 1; model.py:159).
+__device__ __forceinline__ float swiglu(float g, float u) {
+  return (g * __builtin_amdgcn_rcpf(1.f + exp_hw(-g))) * u;
 }
 
-// Four outputs of the packed q/k/v rows col .. col + 3 (col a multiple of 4): qkv_pair for both pairs
-// with whole-run stores.  rp: the position's RoPE row; q: the row's f32 q/k/v.
-__device__ __forceinline__ void qkv_quad(f32x4 v, const float* rp, int col, int H, int KV, float* q, uint16_t* kc,
-                                         uint16_t* vc, int64_t pool, int64_t crow) {
-  const int head = col / kDh, rr = col % kDh;
+// Four outputs of the packed q/k/v rows col .. col + 3 (col a multiple of 4) of row `row`, whose position
+// has the RoPE row rp: q and k pairs are rotated (dims i, i + 32; model.py:110-117), v is stored
+// as projected; f32 q/k/v in natural head-dim order to the row's q (with ea.kvp k and v go to the
+// operand planes instead, row = key), bf16 K/V to the cache row crow (multi_sm_decode.py:179-180).
+__device__ __forceinline__ void qkv_quad(f32x4 v, const float* rp, int col, int row, const EpiArgs& ea, float* q,
+                                         int64_t crow) {
+  const int H = ea.H, KV = ea.KV, head = col / kDh, rr = col % kDh;
+  const int64_t pl = int64_t(KV) * ea.MP * kDh;
   q += head * kDh;
   if (head >= H + KV) {   // v: four consecutive dims
-    *reinterpret_cast<f32x4*>(q + rr) = v;
-    *reinterpret_cast<uint2*>(vc + (int64_t(head - H - KV) * pool + crow) * kDh + rr) =
+    const int g = head - H - KV;
+    if (ea.kvp) {
+      uint32_t hi[2], lo[2];
+      split2(v[0], v[1], hi[0], lo[0]);
+      split2(v[2], v[3], hi[1], lo[1]);
+      uint16_t* vp = ea.kvp + 2 * pl;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t at = v_plane_index(g, row, rr + e, ea.MP);
+        vp[at] = uint16_t(hi[e >> 1] >> (16 * (e & 1)));
+        vp[pl + at] = uint16_t(lo[e >> 1] >> (16 * (e & 1)));
+      }
+    } else {
+      *reinterpret_cast<f32x4*>(q + rr) = v;
+    }
+    *reinterpret_cast<uint2*>(ea.vc + (int64_t(g) * ea.rows.pool + crow) * kDh + rr) =
         make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
     return;
   }
@@ -339,10 +357,23 @@ __device__ __forceinline__ void qkv_quad(f32x4 v, const float* rp, int col, int 
   const f32x2 c = *reinterpret_cast<const f32x2*>(rp + ri), s = *reinterpret_cast<const f32x2*>(rp + kDh / 2 + ri);
   const f32x2 x = {v[0] * c[0] - v[1] * s[0], v[2] * c[1] - v[3] * s[1]};
   const f32x2 y = {v[0] * s[0] + v[1] * c[0], v[2] * s[1] + v[3] * c[1]};
-  *reinterpret_cast<f32x2*>(q + ri) = x;
-  *reinterpret_cast<f32x2*>(q + ri + kDh / 2) = y;
+  if (head < H || !ea.kvp) {
+    *reinterpret_cast<f32x2*>(q + ri) = x;
+    *reinterpret_cast<f32x2*>(q + ri + kDh / 2) = y;
+  }
   if (head >= H) {
-    uint16_t* cp = kc + (int64_t(head - H) * pool + crow) * kDh;
+    const int g = head - H;
+    if (ea.kvp) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        uint32_t hi, lo;
+        split2(half ? y[0] : x[0], half ? y[1] : x[1], hi, lo);
+        uint16_t* kp = ea.kvp + k_plane_index(g, row, ri + half * kDh / 2, ea.MP);
+        *reinterpret_cast<uint32_t*>(kp) = hi;
+        *reinterpret_cast<uint32_t*>(kp + pl) = lo;
+      }
+    }
+    uint16_t* cp = ea.kc + (int64_t(g) * ea.rows.pool + crow) * kDh;
     *reinterpret_cast<uint32_t*>(cp + ri) = pack2(x[0], x[1]);
     *reinterpret_cast<uint32_t*>(cp + ri + kDh / 2) = pack2(y[0], y[1]);
   }
@@ -362,7 +393,7 @@ __device__ __forceinline__ void qkv_quad(f32x4 v, const float* rp, int col, int 
 // h^2 of each row added up from that epilogue's per-column-group partials.  TW as for mx_gemm.
 // EPI: store the outputs, add them to the residual out (tile order; with an act plane also the
 // hi/lo tiles of scale * h and the row's partial sum of h^2 for the next RMSNorm), or finish them
-// in place of mx_swiglu_fin / mx_qkv_fin (column pairs per thread, the same arithmetic).
+// in place of mx_swiglu_fin / mx_qkv_fin (the same arithmetic).
 template <int RT, int CT, int P, int NW, int AM, bool TW, int EPI>
 __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
   static_assert(RT == 1 || (AM >= 1 && TW), "several row tiles per workgroup: tile-order operands");
@@ -544,7 +575,7 @@ __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
         *reinterpret_cast<uint32_t*>(ea.act + at) = hi;
         *reinterpret_cast<uint32_t*>(ea.act + ea.act_plane + at) = lo;
       } else {
-        qkv_quad(v, rp, col, ea.H, ea.KV, ea.qkv + int64_t(row) * g.N, ea.kc, ea.vc, int64_t(ea.rows.pool), crow);
+        qkv_quad(v, rp, col, row, ea, ea.qkv + int64_t(row) * g.N, crow);
       }
     }
     if constexpr (kResid) {   // the wave's columns of the row: four lanes, in a fixed order
@@ -671,10 +702,8 @@ __global__ __launch_bounds__(256) void mx_embed(const uint16_t* emb, const int32
 // Row blockIdx.x: q/k/v = sum_z part[z] (z in order) over the packed q/k/v rows; RoPE on the
 // q and k pairs (packed rows 2i, 2i+1 = dims i, i+32; model.py:110-117) at the row's
 // position; f32 q/k/v in natural head-dim order to qkv; bf16 K/V to the cache.
-__global__ __launch_bounds__(256) void mx_qkv_fin(const float* part, int splits, int M, int H, int KV,
-                                                  const float* rope, Rows rows, uint16_t* kc, uint16_t* vc,
-                                                  float* qkv) {
-  const int m = blockIdx.x, nq = (H + 2 * KV) * kDh;
+__global__ __launch_bounds__(256) void mx_qkv_fin(const float* part, int splits, int M, EpiArgs ea) {
+  const int m = blockIdx.x, nq = (ea.H + 2 * ea.KV) * kDh;
   const int t = blockIdx.y * 256 + threadIdx.x;
   if (t >= nq / 4) return;
   const int col = 4 * t;   // column pairs (col, col + 1) and (col + 2, col + 3), one head
@@ -682,13 +711,8 @@ __global__ __launch_bounds__(256) void mx_qkv_fin(const float* part, int splits,
 #pragma unroll
   for (int z = 0; z < kMaxSplitK; ++z)
     pv[z] = *reinterpret_cast<const float4*>(part + (int64_t(min(z, splits - 1)) * M + m) * nq + col);
-  // the loads that depend on the position (RoPE row, cache row) are issued together, for every
-  // column (a load under a branch is waited for at the join)
-  const int p = row_pos(rows, m);
-  const int64_t crow = cache_row(rows, m, p);
-  const int ri = (col % kDh) >> 1;
-  const float2 cs = *reinterpret_cast<const float2*>(rope + int64_t(p) * kDh + ri);
-  const float2 sn = *reinterpret_cast<const float2*>(rope + int64_t(p) * kDh + kDh / 2 + ri);
+  const int p = row_pos(ea.rows, m);
+  const int64_t crow = cache_row(ea.rows, m, p);
   float4 sv = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int z = 0; z < kMaxSplitK; ++z)
@@ -698,13 +722,7 @@ __global__ __launch_bounds__(256) void mx_qkv_fin(const float* part, int splits,
       sv.z += pv[z].z;
       sv.w += pv[z].w;
     }
-  const int head = col / kDh;
-  float* q = qkv + int64_t(m) * nq + head * kDh;
-  const bool isv = head >= H + KV;
-  const int g = isv ? head - H - KV : head - H;
-  uint16_t* cp = (isv ? vc : kc) + (int64_t(g) * rows.pool + crow) * kDh;
-  qkv_pair(sv.x, sv.y, cs.x, sn.x, col, H, KV, q, cp);
-  qkv_pair(sv.z, sv.w, cs.y, sn.y, col + 2, H, KV, q, cp);
+  qkv_quad(f32x4{sv.x, sv.y, sv.z, sv.w}, ea.rope + int64_t(p) * kDh, col, m, ea, ea.qkv + int64_t(m) * nq, crow);
 }
 
 // Row blockIdx.x: act_f = silu(gate_f) * up_f over the summed partials (gate/up are the packed
@@ -757,10 +775,14 @@ __device__ __forceinline__ float row16_sum(float v) {
 // MFMA operand lanes: A[i][8 (l / 16) ..] = row i = l % 16; B[8 (l / 16) ..][n] with n = l % 16;
 // D: rows 4 (l / 16) + r of column l % 16.
 // The head outputs go to the O projection's input planes at their packed positions, or with
-// natural at their element index (the tile copy's O columns are in natural order).
+// natural at their element index (the tile copy's O columns are in natural order).  K and V come as
+// operand planes from the QKV epilogue, so a chunk is 16 loads of 1 KB and no conversion (reading f32
+// rows took 40 loads of 64-byte segments and eight splits per chunk in every head and query block:
+// 511 rows 15.9 us, now 9.5; 128 rows 6.6, now 4.4).  Eight waves past 128 rows (511 rows of f32: 17.1
+// us with four, 15.9 with eight), four where no wave of eight would have a second chunk.
 template <int NW>
-__global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv, int M, int H, int KV, uint16_t* att,
-                                                            int64_t plane, int ldx, int natural) {
+__global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv, const uint16_t* kvp, int MP, int M, int H,
+                                                                int KV, uint16_t* att, int64_t plane, int natural) {
   constexpr int PS = 36;   // row stride (floats) of a wave's P tile in LDS: 16-byte reads of 16 rows spread over banks
   __shared__ __align__(16) float sp[NW][16 * PS];
   __shared__ float sm[NW][16], sl[NW][16];
@@ -792,38 +814,48 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
     o[r] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   float* P = sp[wv];
+  const int64_t pl = int64_t(KV) * MP * kDh;
+  const uint16_t* kp = kvp + int64_t(g) * MP * kDh + lane * 8;
+  const uint16_t* vp = kp + 2 * pl;
   for (int c = wv; c < nch; c += NW) {
     const int kb = 32 * c;
-    // K rows (B of S: key kb + 16 t + r16, dims 32 ks + 8 kq ..) and V values (B of P V: keys
-    // kb + 8 kq + e, dim 16 dt + r16), all requested before the first MFMA; keys past M read
-    // row M - 1 and are masked
-    float kf[2][2][8], vf[4][8];
+    // K (B of S: key kb + 16 t + r16, dims 32 ks + 8 kq ..) and V (B of P V: keys kb + 8 kq .., dim 16
+    // dt + r16), all requested before the first MFMA, each load one 1 KB piece; keys past M hold
+    // anything: their scores are masked and their V is cleared below
+    uint4 kh[2][2], kl[2][2], vh[4], vl[4];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const float* kr = qkv + int64_t(min(kb + 16 * t + r16, M - 1)) * nqkv + (H + g) * kDh + 8 * kq;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const float4 a = *reinterpret_cast<const float4*>(kr + 32 * ks);
-        const float4 b = *reinterpret_cast<const float4*>(kr + 32 * ks + 4);
-        kf[t][ks][0] = a.x; kf[t][ks][1] = a.y; kf[t][ks][2] = a.z; kf[t][ks][3] = a.w;
-        kf[t][ks][4] = b.x; kf[t][ks][5] = b.y; kf[t][ks][6] = b.z; kf[t][ks][7] = b.w;
+        const uint16_t* kr = kp + ((kb >> 4) + t) * 1024 + ks * 512;
+        kh[t][ks] = *reinterpret_cast<const uint4*>(kr);
+        kl[t][ks] = *reinterpret_cast<const uint4*>(kr + pl);
       }
-    }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float* vr = qkv + int64_t(min(kb + 8 * kq + e, M - 1)) * nqkv + (H + KV + g) * kDh + r16;
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) vf[dt][e] = vr[16 * dt];
+    for (int dt = 0; dt < 4; ++dt) {
+      const uint16_t* vr = vp + (dt * (MP >> 5) + (kb >> 5)) * 512;
+      vh[dt] = *reinterpret_cast<const uint4*>(vr);
+      vl[dt] = *reinterpret_cast<const uint4*>(vr + pl);
     }
     f32x4 s[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        uint4 kh, kl;
-        split8(kf[t][ks], kh, kl);
-        s[t] = mfma3(qh[ks], ql[ks], kh, kl, s[t]);
+      for (int ks = 0; ks < 2; ++ks) s[t] = mfma3(qh[ks], ql[ks], kh[t][ks], kl[t][ks], s[t]);
+    }
+    if (kb + 32 > M) {   // (uniform) V of keys past M: 0 (0 times what the padding holds could be NaN)
+      const int nv = M - kb - 8 * kq;
+      auto clear = [&](uint4& u) {
+        uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = 2 * j + 1 < nv ? w[j] : (2 * j < nv ? w[j] & 0xffffu : 0u);
+        u = make_uint4(w[0], w[1], w[2], w[3]);
+      };
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        clear(vh[dt]);
+        clear(vl[dt]);
       }
     }
     // scale, causal mask, online softmax of rows 4 kq + r over keys kb + 16 t + r16
@@ -834,8 +866,8 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
       const float v0 = (j0 <= i && j0 < M) ? s[0][r] * 0.125f : -INFINITY;
       const float v1 = (j1 <= i && j1 < M) ? s[1][r] * 0.125f : -INFINITY;
       const float mn = fmaxf(m[r], row16_max(fmaxf(v0, v1)));
-      const float p0 = mn == -INFINITY ? 0.f : expf(v0 - mn), p1 = mn == -INFINITY ? 0.f : expf(v1 - mn);
-      const float alpha = m[r] == -INFINITY ? 0.f : expf(m[r] - mn);
+      const float p0 = mn == -INFINITY ? 0.f : exp_hw(v0 - mn), p1 = mn == -INFINITY ? 0.f : exp_hw(v1 - mn);
+      const float alpha = m[r] == -INFINITY ? 0.f : exp_hw(m[r] - mn);
       l[r] = l[r] * alpha + row16_sum(p0 + p1);
       m[r] = mn;
 #pragma unroll
@@ -844,19 +876,15 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
       P[(4 * kq + r) * PS + 16 + r16] = p1;
     }
     __builtin_amdgcn_wave_barrier();
-    uint4 ph, pl;
+    uint4 ph, plo;
     {
       const float4 a = *reinterpret_cast<const float4*>(P + r16 * PS + 8 * kq);
       const float4 b = *reinterpret_cast<const float4*>(P + r16 * PS + 8 * kq + 4);
       const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      split8(x, ph, pl);
+      split8(x, ph, plo);
     }
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      uint4 vh, vl;
-      split8(vf[dt], vh, vl);
-      o[dt] = mfma3(ph, pl, vh, vl, o[dt]);
-    }
+    for (int dt = 0; dt < 4; ++dt) o[dt] = mfma3(ph, plo, vh[dt], vl[dt], o[dt]);
     __builtin_amdgcn_wave_barrier();
   }
   // merge the waves by log-sum-exp
@@ -879,27 +907,33 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
   float L = 0.f, O[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    const float wt = sm[w][qi] == -INFINITY ? 0.f : expf(sm[w][qi] - mx);
+    const float wt = sm[w][qi] == -INFINITY ? 0.f : exp_hw(sm[w][qi] - mx);
     L += sl[w][qi] * wt;
 #pragma unroll
     for (int e = 0; e < 4; ++e) O[e] += so[w][qi][d4 + e] * wt;
   }
-  const int i = q0 + qi;
-  if (i < M)
+  const int i = q0 + qi, el = h * kDh + d4;
+  if (i >= M) return;
+  if (natural) {   // four consecutive positions
+    uint2 hi, lo;
+    split2(O[0] / L, O[1] / L, hi.x, lo.x);
+    split2(O[2] / L, O[3] / L, hi.y, lo.y);
+    const int64_t at = act_index(i, el, d, 0);
+    *reinterpret_cast<uint2*>(att + at) = hi;
+    *reinterpret_cast<uint2*>(att + plane + at) = lo;
+  } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int el = h * kDh + d4 + e;
-      put_split(att + act_index(i, natural ? el : perm_pos(el, d), d, ldx), plane, O[e] / L);
-    }
+    for (int e = 0; e < 4; ++e) put_split(att + act_index(i, perm_pos(el + e, d), d, 0), plane, O[e] / L);
+  }
 }
 
-static void launch_attention_prefill(int M, int H, int KV, hipStream_t s, const float* qkv, uint16_t* att,
-                                     int64_t plane, int natural) {
+static void launch_attention_prefill(int M, int H, int KV, hipStream_t s, const float* qkv, const uint16_t* kvp, int MP,
+                                     uint16_t* att, int64_t plane, int natural) {
   const dim3 grid(H, (M + 15) / 16);
   if (M > 128)
-    hipLaunchKernelGGL(mx_attention_prefill<8>, grid, dim3(512), 0, s, qkv, M, H, KV, att, plane, 0, natural);
+    hipLaunchKernelGGL(mx_attention_prefill<8>, grid, dim3(512), 0, s, qkv, kvp, MP, M, H, KV, att, plane, natural);
   else
-    hipLaunchKernelGGL(mx_attention_prefill<4>, grid, dim3(256), 0, s, qkv, M, H, KV, att, plane, 0, natural);
+    hipLaunchKernelGGL(mx_attention_prefill<4>, grid, dim3(256), 0, s, qkv, kvp, MP, M, H, KV, att, plane, natural);
 }
 
 // Batched decode: row m = blockIdx.x (one sequence at position p = pos(m)) and the GH query heads
@@ -909,7 +943,8 @@ static void launch_attention_prefill(int M, int H, int KV, hipStream_t s, const 
 // reads its K/V): wave w takes the 32-position blocks w, w + 8, ..., the next block's rows requested
 // before the current one's arithmetic.  Lane l reads dims 8 (l % 8) .. + 8 of position 8 i + l / 8, i = 0..3,
 // of K and of V: whole rows, 1 KB per instruction (a lane per position for K and per dim for V took
-// 72 instructions per 64 positions and 64 cache lines per K instruction: 13.9 us for the 24 rows).  The
+// 72 instructions per 64 positions and 64 cache lines per K instruction: 13.9 us for the 24 rows, now
+// 8.2; 5 rows at position 211: 7.4, now 5.4).  The
 // 8 lanes of a position add their partial scores with DPP, so every lane ends up with the weights of
 // exactly the V rows it holds; only (max, sum, output) partials go through LDS at the end.
 constexpr int kAttnWaves = 8;
@@ -1086,8 +1121,10 @@ __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const flo
   }
 }
 
-// Heads per workgroup: as many of a K/V head's as leave about a workgroup per CU (each reads the K/V
-// rows once for its heads; fewer workgroups than CUs cost more than the shared reads save).
+// Four heads of a K/V head per workgroup when that still leaves a workgroup per CU: the K/V rows are
+// then read once for the four (306M, 64 rows: 1004 -> 943 us per step); with fewer workgroups the idle
+// CUs cost more than the shared reads save (24 rows: 803 us with one head, 806 with two, 859 with
+// four).
 static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const float* qkv, const Rows& rows,
                                     const uint16_t* kc, const uint16_t* vc, uint16_t* att, int64_t plane,
                                     int natural) {
@@ -1095,8 +1132,7 @@ static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const f
   auto go = [&](auto k, int gh) {
     hipLaunchKernelGGL(k, dim3(M, H / gh), dim3(64 * kAttnWaves), 0, s, qkv, rows, H, KV, kc, vc, att, plane, 0, natural);
   };
-  if (G % 4 == 0 && M * H / 4 >= 160) go(mx_attention_decode<4>, 4);
-  else if (G % 2 == 0 && M * H / 2 >= 160) go(mx_attention_decode<2>, 2);
+  if (G % 4 == 0 && M * H / 4 >= 256) go(mx_attention_decode<4>, 4);
   else go(mx_attention_decode<1>, 1);
 }
 
@@ -1205,7 +1241,7 @@ __global__ __launch_bounds__(256) void mx_pack_scales(const uint16_t* ln, int d,
 
 // ---------------------------------------------------------------- host side
 struct Layout {
-  size_t h, xn, ssq, qkv, att, act, part, status, rowpos, pages, bytes;
+  size_t h, xn, ssq, qkv, kvp, att, act, part, status, rowpos, pages, bytes;
 };
 
 static size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -1295,6 +1331,7 @@ static size_t part_floats(const msd_config* c, int M) {
 }
 
 static int pad16(int M) { return (M + 15) & ~15; }
+static int pad32(int M) { return (M + 31) & ~31; }
 
 static Layout layout(const msd_config* c, int M) {
   const int d = c->d_model, ff = c->d_ff, nqkv = (c->n_heads + 2 * c->n_kv_heads) * kDh;
@@ -1305,6 +1342,7 @@ static Layout layout(const msd_config* c, int M) {
   L.xn = o;     o += al256(size_t(pad16(M)) * d * 2 * 2);
   L.ssq = o;    o += al256(size_t(M) * (d / 16) * 4);   // partial sums of h^2: at most d / 16 per row
   L.qkv = o;    o += al256(size_t(M) * nqkv * 4);
+  L.kvp = o;    o += al256(size_t(pad32(M)) * c->n_kv_heads * kDh * 2 * 4);   // prefill: K/V operand planes
   L.att = o;    o += al256(size_t(pad16(M)) * d * 2 * 2);
   L.act = o;    o += al256(size_t(pad16(M)) * ff * 2 * 2);
   L.part = o;   o += al256(part_floats(c, M) * 4);
@@ -1422,6 +1460,8 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
   float* h = reinterpret_cast<float*>(ws + L.h);
   uint16_t* xn = reinterpret_cast<uint16_t*>(ws + L.xn);
   float* qkv = reinterpret_cast<float*>(ws + L.qkv);
+  uint16_t* kvp = reinterpret_cast<uint16_t*>(ws + L.kvp);
+  const int MP = pad32(M);
   uint16_t* att = reinterpret_cast<uint16_t*>(ws + L.att);
   uint16_t* act = reinterpret_cast<uint16_t*>(ws + L.act);
   float* part = reinterpret_cast<float*>(ws + L.part);
@@ -1447,6 +1487,16 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
     uint16_t* vc = kc + int64_t(KV) * rows.pool * kDh;
     // activation planes in tile order (ldx 0), the lo planes after the hi planes
     const int64_t pd = int64_t(pad16(M)) * d, pf = int64_t(pad16(M)) * ff;
+    EpiArgs eq{};
+    eq.rope = wt.rope;
+    eq.rows = rows;
+    eq.kc = kc;
+    eq.vc = vc;
+    eq.qkv = qkv;
+    eq.H = H;
+    eq.KV = KV;
+    eq.kvp = prefill ? kvp : nullptr;
+    eq.MP = MP;
     if (tw) {
       // Five kernels per layer over the tile copy, h in packed order: QKV with RMSNorm1 folded in
       // and q/k/v, RoPE and the cache rows in its epilogue; attention; O adding to h and writing
@@ -1454,19 +1504,11 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
       // adding to h and writing the next layer's RMSNorm1 input planes.
       const uint16_t* Tl = wt.tiles + int64_t(l) * tile_layer_elems(cfg);
       const bool last = l + 1 == cfg->n_layers;
-      EpiArgs eq{};
-      eq.rope = wt.rope;
-      eq.rows = rows;
-      eq.kc = kc;
-      eq.vc = vc;
-      eq.qkv = qkv;
-      eq.H = H;
-      eq.KV = KV;
       if ((err = gemm(xn, pd, 0, Tl, true, M, nqkv, d, nullptr, 0, 1, s, true, kEpiQkv, &eq, ssq, l == 0 ? 1 : cg_d)) !=
           hipSuccess)
         break;
       if (prefill)
-        launch_attention_prefill(M, H, KV, s, qkv, att, pd, 1);
+        launch_attention_prefill(M, H, KV, s, qkv, kvp, MP, att, pd, 1);
       else
         launch_attention_decode(M, H, KV, s, qkv, rows, kc, vc, att, pd, 1);
       EpiArgs en{};   // the next RMSNorm's input planes and partial sums of h^2
@@ -1490,10 +1532,9 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
     }
     hipLaunchKernelGGL(mx_norm, dim3(M), dim3(kNormThreads), 0, s, h, part, pending, M, d, Wl, xn, pd, 0, 0, 0);
     if ((err = gemm(xn, pd, 0, Wl + off_qkv, false, M, nqkv, d, part, nqkv, sq, s)) != hipSuccess) break;
-    hipLaunchKernelGGL(mx_qkv_fin, dim3(M, (nqkv / 4 + 255) / 256), dim3(256), 0, s, part, sq, M, H, KV, wt.rope, rows,
-                       kc, vc, qkv);
+    hipLaunchKernelGGL(mx_qkv_fin, dim3(M, (nqkv / 4 + 255) / 256), dim3(256), 0, s, part, sq, M, eq);
     if (prefill)
-      launch_attention_prefill(M, H, KV, s, qkv, att, pd, 0);
+      launch_attention_prefill(M, H, KV, s, qkv, kvp, MP, att, pd, 0);
     else
       launch_attention_decode(M, H, KV, s, qkv, rows, kc, vc, att, pd, 0);
     if ((err = gemm(att, pd, 0, Wl + off_o, false, M, d, d, part, d, so, s)) != hipSuccess) break;
