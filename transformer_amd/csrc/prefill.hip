@@ -413,13 +413,15 @@ __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
   const int ctn = min(CT, n16 - CT * c);   // column tiles of this group (the last group may be short)
   const int r16 = lane & 15, kq = 8 * (lane >> 4);
   const int S = g.K / kBK;
-  // rows past M read row M - 1 (row layout) or whatever their tile holds (a row tile past the
-  // last reads the last): an MFMA row only feeds its own output row, which is not stored
+  // rows past M read row M - 1 (a row tile past the last reads the last): an MFMA row only feeds its
+  // own output row, which is not stored, and a short tile costs only its rows' cache lines
   const uint16_t* ar[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-    ar[rt] = AM >= 1 ? g.A + (int64_t(min(RT * t + rt, T - 1)) * S * 64 + lane) * 8
+  for (int rt = 0; rt < RT; ++rt) {
+    const int tile = min(RT * t + rt, T - 1);
+    ar[rt] = AM >= 1 ? g.A + (int64_t(tile) * S * 64 + min(r16, g.M - 1 - 16 * tile) + 16 * (lane >> 4)) * 8
                      : g.A + int64_t(min(m0 + r16, g.M - 1)) * g.lda + kq;
+  }
   const uint16_t* wr = TW ? g.W + (int64_t(n0 >> 4) * S * 64 + lane) * 8 : g.W + int64_t(n0 + r16) * g.K + kq;
   // element offsets of step ks and of column tile ct
   const int64_t astep = AM >= 1 ? 512 : kBK, wstep = TW ? 512 : kBK;
@@ -669,10 +671,9 @@ __global__ __launch_bounds__(256) void mx_embed(const uint16_t* emb, const int32
   __shared__ float red[4];
   const int m = blockIdx.x;
   int t = tokens[m];
-  if (t < 0 || t >= V) {
-    if (threadIdx.x == 0) atomicOr(status, 2);
-    t = 0;
-  }
+  const bool bad = t < 0 || t >= V;
+  if (threadIdx.x == 0) status[m] = bad ? 2 : 0;
+  if (bad) t = 0;
   constexpr int NE = kMaxRows / 256;   // every load issued before the first store
   uint16_t e[NE];
 #pragma unroll
@@ -1136,10 +1137,152 @@ static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const f
   else go(mx_attention_decode<1>, 1);
 }
 
-// argmax of each row of logits (lowest index on ties): out[2*row] = index, out[2*row+1] = status
+// Tied logits of several rows: out[m][v] = sum_k x[m][k] W[v][k] with x the final norm's hi/lo planes
+// (rows of K) and W the embedding rows.  A workgroup of four waves owns 128 vocabulary rows x TOK rows;
+// K advances 32 at a time through a ring of S LDS stages filled by direct DMA (W rows, hi rows, lo
+// rows of 64 bytes; piece c of row r at position c ^ ((r >> 2) & 3), which makes the fragment reads
+// conflict-free).  Each output sums K steps in order, hi then lo, on 16 x 16 x 32 MFMAs as mx_gemm
+// does, so the last row's logits are bitwise the same whether one row or every row is requested.
+// mx_gemm's fragment loads of the row layout are 64 requests of 16 bytes each and bound it: 203 rows
+// of d 768 93 us, here 32.5; 24 rows of d 1024 33 us, here 15.8 (65 MB: 13 us at the card's
+// copy rate).  TOK: 32 and 64 where the rows fit, else 128 (LDS reads per MFMA fall with TOK).
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+template <int RB, int CB>
+struct LogitFrags {
+  u32x4v w[RB], x[2][CB];
+};
+// the fragment reads of a stage and their wait in one block
+__device__ __forceinline__ void logit_reads(LogitFrags<2, 2>& f, uint32_t a, uint32_t b, uint32_t bl) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "ds_read_b128 %0, %6\nds_read_b128 %1, %6 offset:1024\n"
+      "ds_read_b128 %2, %7\nds_read_b128 %3, %7 offset:1024\n"
+      "ds_read_b128 %4, %8\nds_read_b128 %5, %8 offset:1024\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(f.w[0]), "=&v"(f.w[1]), "=&v"(f.x[0][0]), "=&v"(f.x[0][1]), "=&v"(f.x[1][0]), "=&v"(f.x[1][1])
+      : "v"(a), "v"(b), "v"(bl));
+#endif
+}
+__device__ __forceinline__ void logit_reads(LogitFrags<4, 2>& f, uint32_t a, uint32_t b, uint32_t bl) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "ds_read_b128 %0, %8\nds_read_b128 %1, %8 offset:1024\n"
+      "ds_read_b128 %2, %8 offset:2048\nds_read_b128 %3, %8 offset:3072\n"
+      "ds_read_b128 %4, %9\nds_read_b128 %5, %9 offset:1024\n"
+      "ds_read_b128 %6, %10\nds_read_b128 %7, %10 offset:1024\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(f.w[0]), "=&v"(f.w[1]), "=&v"(f.w[2]), "=&v"(f.w[3]), "=&v"(f.x[0][0]), "=&v"(f.x[0][1]),
+        "=&v"(f.x[1][0]), "=&v"(f.x[1][1])
+      : "v"(a), "v"(b), "v"(bl));
+#endif
+}
+__device__ __forceinline__ void logit_reads(LogitFrags<4, 4>& f, uint32_t a, uint32_t b, uint32_t bl) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "ds_read_b128 %0, %12\nds_read_b128 %1, %12 offset:1024\n"
+      "ds_read_b128 %2, %12 offset:2048\nds_read_b128 %3, %12 offset:3072\n"
+      "ds_read_b128 %4, %13\nds_read_b128 %5, %13 offset:1024\n"
+      "ds_read_b128 %6, %13 offset:2048\nds_read_b128 %7, %13 offset:3072\n"
+      "ds_read_b128 %8, %14\nds_read_b128 %9, %14 offset:1024\n"
+      "ds_read_b128 %10, %14 offset:2048\nds_read_b128 %11, %14 offset:3072\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(f.w[0]), "=&v"(f.w[1]), "=&v"(f.w[2]), "=&v"(f.w[3]), "=&v"(f.x[0][0]), "=&v"(f.x[0][1]),
+        "=&v"(f.x[0][2]), "=&v"(f.x[0][3]), "=&v"(f.x[1][0]), "=&v"(f.x[1][1]), "=&v"(f.x[1][2]), "=&v"(f.x[1][3])
+      : "v"(a), "v"(b), "v"(bl));
+#endif
+}
+// at most n (< D) stages of NI DMA instructions outstanding, then the workgroup's barrier (a bare one:
+// __syncthreads would wait for every outstanding DMA)
+template <int NI, int D>
+__device__ __forceinline__ void wait_stage_barrier(int n) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (D > 1) {
+    if (n < D - 1) return wait_stage_barrier<NI, D - 1>(n);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)\ns_barrier" ::"n"((D - 1) * NI) : "memory");
+#endif
+}
+constexpr int kLogitRows = 128;   // vocabulary rows per workgroup
+template <int TOK>
+__global__ __launch_bounds__(256) void mx_logits(const uint16_t* X, int64_t plane, const uint16_t* W, int M, int V, int K,
+                                                 float* out) {
+  constexpr int GM = TOK == 32 ? 4 : 2, GN = 4 / GM;              // waves over vocabulary x rows
+  constexpr int RB = kLogitRows / GM / 16, CB = TOK / GN / 16;    // 16-row fragments per wave
+  constexpr int SD = (kLogitRows + 2 * TOK) * 64, NI = SD / 1024 / 4, S = TOK == 128 ? 3 : (TOK == 64 ? 4 : 6), D = S - 1;
+  __shared__ __align__(1024) uint8_t ring[S * SD];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wv / GN, wn = wv % GN;
+  // (each XCD takes a contiguous range of the tiles, row tiles innermost, so W reaches its L2 once)
+  const int MT = (M + TOK - 1) / TOK, xcd = blockIdx.x & 7, per = gridDim.x >> 3, rest = gridDim.x & 7;
+  const int id = xcd * per + min(xcd, rest) + (blockIdx.x >> 3);
+  const int v0 = kLogitRows * (id / MT), m0 = TOK * (id % MT);
+  // instruction u of this wave fills the 1 KB piece wv + 4 u of a stage: 16 rows of W, hi or lo (rows
+  // past the last read the last)
+  const uint16_t* src[NI];
+#pragma unroll
+  for (int u = 0; u < NI; ++u) {
+    const int q = wv + 4 * u, x = q - kLogitRows / 16;
+    const int r = 16 * (x < 0 ? q : x % (TOK / 16)) + (lane >> 2);
+    const int piece = (lane & 3) ^ ((r >> 2) & 3);
+    src[u] = (x < 0 ? W + int64_t(min(v0 + r, V - 1)) * K
+                    : X + (x < TOK / 16 ? 0 : plane) + int64_t(min(m0 + r, M - 1)) * K) + 8 * piece;
+  }
+  auto dma = [&](int kt) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    uint8_t* st = ring + (kt % S) * SD;
+#pragma unroll
+    for (int u = 0; u < NI; ++u)
+      __builtin_amdgcn_global_load_lds(src[u] + kt * kBK,
+                                       (__attribute__((address_space(3))) void*)(st + 1024 * (wv + 4 * u)), 16, 0, 0);
+#endif
+  };
+  const int KT = K / kBK;
+  for (int s = 0; s < D && s < KT; ++s) dma(s);
+  f32x4 acc[RB][CB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int r16 = lane & 15, kq = lane >> 4;
+  const uint32_t base = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)ring));
+  const uint32_t fr = base + r16 * 64 + ((kq ^ ((r16 >> 2) & 3)) << 4);
+  for (int kt = 0; kt < KT; ++kt) {
+    // stage kt landed for every wave, and stage kt - 1's reads done: its slot takes stage kt + D
+    wait_stage_barrier<NI, D>(min(KT, kt + D) - kt - 1);
+    if (kt + D < KT) dma(kt + D);
+    const uint32_t st = fr + (kt % S) * SD;
+    LogitFrags<RB, CB> f;
+    const uint32_t b = st + (kLogitRows + wn * 16 * CB) * 64;
+    logit_reads(f, st + wm * RB * 1024, b, b + TOK * 64);
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        const bf16x8 w = __builtin_bit_cast(bf16x8, f.w[i]);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8, f.x[0][j]), acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8, f.x[1][j]), acc[i][j], 0, 0, 0);
+      }
+  }
+  // a lane holds four consecutive vocabulary ids of one row (V is a multiple of 16)
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int m = m0 + 16 * (wn * CB + j) + r16;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const int v = v0 + 16 * (wm * RB + i) + 4 * kq;
+      if (m < M && v < V) *reinterpret_cast<f32x4*>(out + int64_t(m) * V + v) = acc[i][j];
+    }
+  }
+}
+
+// argmax of each row of logits (lowest index on ties): out[2*row] = index, out[2*row+1] = the pass's
+// status, i.e. every row's flags (status[0..nflags): tokens by mx_embed, then positions by
+// mx_sanitize_rows) together.  copy (optional, one row): the row's logits again.
 __global__ __launch_bounds__(1024) void mx_argmax(const float* logits, int V, int ld, int32_t* out,
-                                                  const int32_t* status) {
+                                                  const int32_t* status, int nflags, float* copy) {
   __shared__ uint64_t red[16];
+  int flags = 0;
+  for (int i = threadIdx.x; i < nflags; i += 1024) flags |= status[i];
   const float* lr = logits + int64_t(blockIdx.x) * ld;
   uint64_t best = 0;
   constexpr int kBatch = 16;   // loads in flight per thread (clamped, so none sits under a branch)
@@ -1150,6 +1293,7 @@ __global__ __launch_bounds__(1024) void mx_argmax(const float* logits, int V, in
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int j = j0 + 1024 * u;
+      if (copy && j < V) copy[j] = x[u];
       uint32_t b = __float_as_uint(x[u]);
       b = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
       const uint64_t key = (uint64_t(b) << 32) | uint64_t(0xffffffffu - uint32_t(j));
@@ -1161,12 +1305,12 @@ __global__ __launch_bounds__(1024) void mx_argmax(const float* logits, int V, in
     best = w > best ? w : best;
   }
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
-  __syncthreads();
+  const int tok = __syncthreads_or(flags & 2), pos = __syncthreads_or(flags & 4);
   if (threadIdx.x == 0) {
     uint64_t b = red[0];
     for (int i = 1; i < 16; ++i) b = red[i] > b ? red[i] : b;
     out[2 * blockIdx.x] = int32_t(0xffffffffu - uint32_t(b & 0xffffffffu));
-    out[2 * blockIdx.x + 1] = *status;
+    out[2 * blockIdx.x + 1] = (tok ? 2 : 0) | (pos ? 4 : 0);
   }
 }
 
@@ -1198,7 +1342,7 @@ __global__ void mx_sanitize_rows(const int32_t* pos, int fixed_pos, const int32_
     }
   }
   if (pos_out) pos_out[m] = p;
-  if (bad) atomicOr(status, 4);
+  status[m] = bad ? 4 : 0;
 }
 
 // One 16-byte piece per thread of the tile copy of an N x K matrix W (rows in packed order): piece
@@ -1346,7 +1490,7 @@ static Layout layout(const msd_config* c, int M) {
   L.att = o;    o += al256(size_t(pad16(M)) * d * 2 * 2);
   L.act = o;    o += al256(size_t(pad16(M)) * ff * 2 * 2);
   L.part = o;   o += al256(part_floats(c, M) * 4);
-  L.status = o; o += 256;
+  L.status = o; o += al256(size_t(M) * 2 * 4);   // flags: each row's token, then each row's position
   L.rowpos = o; o += al256(size_t(M) * 4);
   L.pages = o;  o += al256(size_t(M) * ((c->context_len + kPage - 1) / kPage) * 4);
   L.bytes = o;
@@ -1425,6 +1569,20 @@ static hipError_t gemm(const uint16_t* A, int64_t a_plane, int lda, const uint16
   const dim3 grid(N / kBN, (M + bm - 1) / bm, splits);
   if (am == 1) launch_splitk<true, false>(bm, grid, s, g);
   else launch_splitk<false, false>(bm, grid, s, g);
+  return hipGetLastError();
+}
+
+static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Tied logits of M rows (planes [M][K], the lo plane M K further).  One row: mx_gemm (15.4 us for the
+// 306M's; its weight rows come straight to the registers), which 5 rows already make slower (17.8).
+static hipError_t launch_logits(const uint16_t* x, const uint16_t* W, int M, int V, int K, float* out, hipStream_t s) {
+  const int64_t plane = int64_t(M) * K;
+  const int nv = (V + kLogitRows - 1) / kLogitRows;
+  if (M == 1 || !aligned16(out)) return gemm(x, plane, K, W, false, M, V, K, out, V, 1, s, false);
+  if (M <= 32) hipLaunchKernelGGL(mx_logits<32>, dim3(nv), dim3(256), 0, s, x, plane, W, M, V, K, out);
+  else if (M <= 64) hipLaunchKernelGGL(mx_logits<64>, dim3(nv), dim3(256), 0, s, x, plane, W, M, V, K, out);
+  else hipLaunchKernelGGL(mx_logits<128>, dim3(nv * ((M + 127) / 128)), dim3(256), 0, s, x, plane, W, M, V, K, out);
   return hipGetLastError();
 }
 
@@ -1548,14 +1706,6 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
   return pending;
 }
 
-static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
-__global__ void mx_clear_status(int32_t* status) { *status = 0; }
-__global__ void mx_copy_f32(const float* src, float* dst, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
-
 // ---- Replaying a pass's launches from a graph (opt-in) ----
 // A pass is ~130 dependent launches; enqueueing them costs the host ~0.35 ms per pass (306M),
 // replaying them from a graph ~0.07 ms.  The device runs the replay ~1 % slower (128-token
@@ -1565,7 +1715,6 @@ __global__ void mx_copy_f32(const float* src, float* dst, int n) {
 // contents are read when the kernels run, so a replay with new tokens or weights in the same
 // buffers is exact.  Captured on a private stream of the device (capture runs nothing) and launched
 // on the caller's stream; a stream that is itself being captured gets the launches directly.
-// The status word is cleared by a kernel, not a memset node.
 constexpr size_t kGraphCache = 16;   // graphs kept per process (least recently used is dropped)
 
 struct GraphEntry {
@@ -1707,10 +1856,9 @@ static int32_t prefill_impl(const msd_config* cfg, const Weights& wt, const int3
   float* part = reinterpret_cast<float*>(ws + L.part);
   int32_t* status = reinterpret_cast<int32_t*>(ws + L.status);
   int32_t* pages = reinterpret_cast<int32_t*>(ws + L.pages);
-  hipLaunchKernelGGL(mx_clear_status, dim3(1), dim3(1), 0, s, status);
   if (page_table)
     hipLaunchKernelGGL(mx_sanitize_rows, dim3(1), dim3(64), 0, s, nullptr, start + M - 1, page_table, 1, max_pages,
-                       cfg->context_len, pool_pages, nullptr, pages, status);
+                       cfg->context_len, pool_pages, nullptr, pages, status + M);
   Rows rows{M, nullptr, 0, page_table ? pages : nullptr, max_pages, page_table ? pool_pages * kPage : cfg->context_len,
             start};
   const int packed = wt.tiles != nullptr;   // the tile path keeps h in packed order
@@ -1725,16 +1873,14 @@ static int32_t prefill_impl(const msd_config* cfg, const Weights& wt, const int3
   const int r0 = logits_all ? 0 : M - 1, nr = M - r0;
   hipLaunchKernelGGL(mx_norm, dim3(nr), dim3(kNormThreads), 0, s, h, part, pending, M, d, wt.lnf, xn,
                      int64_t(nr) * d, r0, d, packed);
-  if (gemm(xn, int64_t(nr) * d, d, wt.outp, false, nr, V, d, logits_all ? logits_all : logits_last, V, 1, s, false) !=
-      hipSuccess)
-    return MSD_E_HIP;
+  if (launch_logits(xn, wt.outp, nr, V, d, logits_all ? logits_all : logits_last, s) != hipSuccess) return MSD_E_HIP;
   const float* last = logits_all ? logits_all + int64_t(M - 1) * V : logits_last;
-  if (logits_all && last != logits_last)
-    hipLaunchKernelGGL(mx_copy_f32, dim3((V + 255) / 256), dim3(256), 0, s, last, logits_last, V);
+  const int nflags = M + (page_table ? 1 : 0);
   if (argmax_all)   // every row (next_token points at the last row's pair)
-    hipLaunchKernelGGL(mx_argmax, dim3(M), dim3(1024), 0, s, logits_all, V, V, argmax_all, status);
-  else
-    hipLaunchKernelGGL(mx_argmax, dim3(1), dim3(1024), 0, s, logits_last, V, V, next_token, status);
+    hipLaunchKernelGGL(mx_argmax, dim3(M), dim3(1024), 0, s, logits_all, V, V, argmax_all, status, nflags, nullptr);
+  if (!argmax_all || last != logits_last)
+    hipLaunchKernelGGL(mx_argmax, dim3(1), dim3(1024), 0, s, last, V, V, next_token, status, nflags,
+                       last != logits_last ? logits_last : nullptr);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_E_HIP;
   });
 }
@@ -1864,9 +2010,8 @@ extern "C" int32_t msd_batch_decode_step(const msd_config* cfg, const void* toke
   int32_t* status = reinterpret_cast<int32_t*>(ws + L.status);
   int32_t* rowpos = reinterpret_cast<int32_t*>(ws + L.rowpos);
   int32_t* pages = reinterpret_cast<int32_t*>(ws + L.pages);
-  hipLaunchKernelGGL(mx_clear_status, dim3(1), dim3(1), 0, s, status);
   hipLaunchKernelGGL(mx_sanitize_rows, dim3((M + 255) / 256), dim3(256), 0, s, positions, 0, page_tables, M, max_pages,
-                     cfg->context_len, pool_pages, rowpos, pages, status);
+                     cfg->context_len, pool_pages, rowpos, pages, status + M);
   Rows rows{M, rowpos, 1, pages, max_pages, pool_pages * kPage, 0};
   const int packed = wt.tiles != nullptr;
   // with the tile copy also the first layer's RMSNorm1 input planes and sums of h^2
@@ -1878,8 +2023,8 @@ extern "C" int32_t msd_batch_decode_step(const msd_config* cfg, const void* toke
   if (err != hipSuccess) return MSD_E_HIP;
   hipLaunchKernelGGL(mx_norm, dim3(M), dim3(kNormThreads), 0, s, h, part, pending, M, d, wt.lnf, xn, int64_t(M) * d, 0,
                      d, packed);
-  if (gemm(xn, int64_t(M) * d, d, wt.outp, false, M, V, d, logits, V, 1, s, false) != hipSuccess) return MSD_E_HIP;
-  hipLaunchKernelGGL(mx_argmax, dim3(M), dim3(1024), 0, s, logits, V, V, next_tokens, status);
+  if (launch_logits(xn, wt.outp, M, V, d, logits, s) != hipSuccess) return MSD_E_HIP;
+  hipLaunchKernelGGL(mx_argmax, dim3(M), dim3(1024), 0, s, logits, V, V, next_tokens, status, 2 * M, nullptr);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_E_HIP;
   });
 }
