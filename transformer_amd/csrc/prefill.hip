@@ -1427,8 +1427,9 @@ static RowsTile rows_tile(int M, int N, int K, int max_groups = 0) {
   for (const RowsTile& t : kRowsTiles) {
     const int C = (n16 + t.ct - 1) / t.ct;
     if (max_groups && C > max_groups) continue;
-    // one column of tiles: 8 waves where a wave of 4 would walk a long K or the CU is otherwise idle
-    if (t.rt * t.ct == 1 && (t.nw == 8) != (S >= 64 || T == 1)) continue;
+    // single tiles: 8 waves for one row tile, and for a long K until the grid fills the chip (down
+    // projection, 8 / 4 waves: 5 rows 5.3 / 5.7 us, 24 rows 5.4 / 5.5, 64 rows 6.8 / 5.8)
+    if (t.rt * t.ct == 1 && (t.nw == 8) != (T == 1 || (S >= 64 && T < 4))) continue;
     const int wg = ((T + t.rt - 1) / t.rt) * C;
     const double step = 0.013 * (2 * t.rt + t.ct) * S, epi = 0.19 * t.rt * t.ct;
     const double cost = t.rt * t.ct <= 12 ? std::max(1.0, wg / 256.0) * step + epi + (wg > 256 ? 0.4 : 0.0)
@@ -1516,12 +1517,13 @@ static void launch_rows_packed(int ct, int grid, hipStream_t s, const GemmArgs& 
   }
 }
 
-// K steps in flight per wave: 4 while the tile leaves the registers for it
+// K steps in flight per wave: 4 while the tile leaves the registers for it (single residual tiles of 4
+// waves: 8, all of a 1024-wide projection; more gained nothing elsewhere)
 template <int AM, int EPI, int I = 0>
 static void launch_rows_tiles(const RowsTile& t, int grid, hipStream_t s, const GemmArgs& g) {
   constexpr RowsTile k = kRowsTiles[I];
   if (t.rt == k.rt && t.ct == k.ct && t.nw == k.nw) {
-    constexpr int P = k.rt == 1 && k.ct <= 4 ? 4 : (k.rt * k.ct <= 6 ? 3 : 2);
+    constexpr int P = k.rt * k.ct == 1 && k.nw == 4 && EPI == kEpiResid ? 8 : k.rt == 1 && k.ct <= 4 ? 4 : (k.rt * k.ct <= 6 ? 3 : 2);
     hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI>), dim3(grid), dim3(64 * k.nw), 0, s, g);
   } else if constexpr (I + 1 < int(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))) {
     launch_rows_tiles<AM, EPI, I + 1>(t, grid, s, g);
