@@ -33,6 +33,12 @@ extern "C" {
  * most 64 MiB or one n_rows x d_model, whichever is more).  MSD_E_CONFIG for an unsupported shape. */
 int64_t msd_xent_workspace_bytes(int32_t n_rows, int32_t vocab, int32_t d_model, int32_t chunk);
 
+/* Targets for the calls below: int32 copies (out, n_rows) of n_rows int32 (bytes_each 4) or int64
+ * (bytes_each 8, low words) device targets, and in *status (written, not accumulated) 4 if any is
+ * outside [0, vocab), else 0.  For callers that hold int64 targets or check them before the forward. */
+int32_t msd_xent_targets(const void* targets, int32_t bytes_each, int32_t n_rows, int32_t vocab, int32_t* out,
+                         int32_t* status, void* stream);
+
 /* Forward.  loss: device f32 scalar, the mean over rows of lse - target logit; lse: device f32
  * (n_rows), each row's logsumexp, kept for the backward (the reference recomputes it,
  * model.py:331-340). */

@@ -622,6 +622,21 @@ __global__ __launch_bounds__(256) void xent_sum_parts(const float* part, int spl
       make_uint2(f2bf(s.x) | (uint32_t(f2bf(s.y)) << 16), f2bf(s.z) | (uint32_t(f2bf(s.w)) << 16));
 }
 
+// Targets as int32 (from int32, or the low words of int64) and, in status[0], whether any is outside
+// [0, V).  One workgroup: it needs no cleared status word and is done long before the logits GEMM,
+// so a caller that checks waits for this kernel only.
+template <typename I>
+__global__ __launch_bounds__(1024) void xent_targets(const I* targets, int n, int V, int32_t* out, int32_t* status) {
+  bool bad = false;
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const int32_t t = int32_t(targets[i]);
+    out[i] = t;
+    bad |= t < 0 || t >= V;
+  }
+  bad = __syncthreads_or(bad);
+  if (threadIdx.x == 0) status[0] = bad ? kStatusTarget : 0;
+}
+
 // lse of each token from its vocabulary tiles' (max, sum); loss term lse - target logit.  16 lanes
 // per token (a block of 256 threads takes 16 tokens): lane u merges tiles u, u + 16, ... in order,
 // then the 16 partials are merged pairwise in a fixed tree (lanes u, u ^ 1, u ^ 2, u ^ 4, u ^ 8)
@@ -768,6 +783,20 @@ using namespace mxe;
 extern "C" int64_t msd_xent_workspace_bytes(int32_t n_rows, int32_t vocab, int32_t d_model, int32_t chunk) {
   if (!shape_ok(n_rows, vocab, d_model)) return MSD_E_CONFIG;
   return layout(n_rows, vocab, d_model, plan(n_rows, vocab, d_model, chunk)).bytes;
+}
+
+extern "C" int32_t msd_xent_targets(const void* targets, int32_t bytes_each, int32_t n_rows, int32_t vocab, int32_t* out,
+                                    int32_t* status, void* stream) {
+  if (n_rows < 1 || vocab < 1) return MSD_E_CONFIG;
+  if (!targets || !out || !status || (bytes_each != 4 && bytes_each != 8)) return MSD_E_ARG;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (bytes_each == 8)
+    hipLaunchKernelGGL(xent_targets<int64_t>, dim3(1), dim3(1024), 0, s, static_cast<const int64_t*>(targets), n_rows, vocab,
+                       out, status);
+  else
+    hipLaunchKernelGGL(xent_targets<int32_t>, dim3(1), dim3(1024), 0, s, static_cast<const int32_t*>(targets), n_rows, vocab,
+                       out, status);
+  return hipGetLastError() == hipSuccess ? MSD_OK : MSD_E_HIP;
 }
 
 extern "C" int32_t msd_xent_forward(const void* h, const void* weight, const int32_t* targets, int32_t n_rows,

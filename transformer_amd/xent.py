@@ -10,7 +10,7 @@ bf16 parameters), targets integer (N,).  The result is the mean cross-entropy as
 tensor with autograd: its backward gives grad_h and grad_weight in the inputs' dtype (bf16), as
 the reference's backward casts them (model.py:361).
 
-What runs (``msd_xent_forward`` / ``msd_xent_backward``, ``csrc/xent.hip``): the forward streams
+What runs (``msd_xent_targets`` / ``msd_xent_forward`` / ``msd_xent_backward``, ``csrc/xent.hip``): the forward streams
 the whole vocabulary through one MFMA GEMM whose epilogue keeps only each row's running
 (max, sum of exponentials), so no logits are stored; the per-row logsumexp is kept for the
 backward.  The backward runs chunk by chunk over the vocabulary (at least ``chunk_size`` columns;
@@ -66,21 +66,31 @@ class FusedCrossEntropy(torch.autograd.Function):
     def forward(ctx, h, weight, targets, chunk_size, check_targets):
         _check_inputs(h, weight, targets)
         h, weight = h.contiguous(), weight.contiguous()
-        tg = targets.to(torch.int32).contiguous()
         N, d = h.shape
         V = weight.shape[0]
         chunk = int(chunk_size)
         ws = _Workspace.get(h.device, N, V, d, chunk)
         loss = torch.empty((), dtype=torch.float32, device=h.device)
         lse = torch.empty(N, dtype=torch.float32, device=h.device)
-        status = torch.zeros(1, dtype=torch.int32, device=h.device)
+        # int32 targets and the status word behind them
+        tg = torch.empty(N + 1, dtype=torch.int32, device=h.device)
+        raw = (targets if targets.dtype in (torch.int32, torch.int64) else targets.to(torch.int32)).contiguous()
         s = torch.cuda.current_stream(h.device)
+        stream = ctypes.c_void_p(s.cuda_stream)
+        status = tg.data_ptr() + 4 * N
+        _lib.check(_lib.lib().msd_xent_targets(raw.data_ptr(), raw.element_size(), N, V, tg.data_ptr(), status, stream),
+                   "msd_xent_targets")
+        if check_targets:   # the copy back waits for the targets only, while the logits GEMM runs
+            host = torch.empty(1, dtype=torch.int32, pin_memory=True)
+            host.copy_(tg[N:], non_blocking=True)
+            copied = s.record_event()
         rc = _lib.lib().msd_xent_forward(h.data_ptr(), weight.data_ptr(), tg.data_ptr(), N, V, d, ws.data_ptr(),
-                                         loss.data_ptr(), lse.data_ptr(), status.data_ptr(),
-                                         ctypes.c_void_p(s.cuda_stream))
+                                         loss.data_ptr(), lse.data_ptr(), status, stream)
         _lib.check(rc, "msd_xent_forward")
-        if check_targets and int(status.item()) & STATUS_BAD_TARGET:
-            raise ValueError(f"a target id outside [0, {V})")
+        if check_targets:
+            copied.synchronize()
+            if int(host) & STATUS_BAD_TARGET:
+                raise ValueError(f"a target id outside [0, {V})")
         ctx.save_for_backward(h, weight, tg, lse)
         ctx.chunk = chunk
         return loss
@@ -94,21 +104,21 @@ class FusedCrossEntropy(torch.autograd.Function):
         gl = g.detach().to(torch.float32).reshape(1).contiguous()
         grad_h = torch.empty_like(h)
         grad_w = torch.empty_like(weight)
-        status = torch.zeros(1, dtype=torch.int32, device=h.device)
         s = torch.cuda.current_stream(h.device)
         rc = _lib.lib().msd_xent_backward(h.data_ptr(), weight.data_ptr(), tg.data_ptr(), lse.data_ptr(),
                                           gl.data_ptr(), N, V, d, ctx.chunk, ws.data_ptr(), grad_h.data_ptr(),
-                                          grad_w.data_ptr(), status.data_ptr(), ctypes.c_void_p(s.cuda_stream))
+                                          grad_w.data_ptr(), tg.data_ptr() + 4 * N, ctypes.c_void_p(s.cuda_stream))
         _lib.check(rc, "msd_xent_backward")
-        ctx.keep = (gl, status)
+        ctx.keep = gl
         return grad_h, grad_w, None, None, None
 
 
 def fused_cross_entropy(h, weight, targets, chunk_size=4096, check_targets=True):
     """model.py:305-312: mean cross-entropy of h @ weight.T against targets without storing the
     logits.  h (N, d), weight (V, d) bf16 on the GPU, targets (N,) integers in [0, V).
-    ``check_targets`` reads the kernel's status back (one small synchronising copy) and raises
-    ValueError for ids outside the vocabulary (they are used as 0 otherwise)."""
+    ``check_targets`` reads the targets' status back (one small synchronising copy, which waits for
+    the targets but not for the loss) and raises ValueError for ids outside the vocabulary (they
+    are used as 0 otherwise)."""
     return FusedCrossEntropy.apply(h, weight, targets, chunk_size, check_targets)
 
 
