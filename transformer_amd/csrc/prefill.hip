@@ -792,7 +792,11 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
   const int r16 = lane & 15, kq = lane >> 4;
   const int h = blockIdx.x, g = h / (H / KV);
   const int nqkv = (H + 2 * KV) * kDh, d = H * kDh;
-  const int q0 = blockIdx.y * 16;
+  // the first half of the grid takes the later query blocks, latest first, the second half the earlier
+  // ones, earliest first: two workgroups half a grid apart, which tend to share a CU, then have
+  // about the same number of chunks together on every CU (511 rows: 9.5 -> 8.0 us)
+  const int half = gridDim.y / 2;
+  const int q0 = 16 * (int(blockIdx.y) < half ? int(gridDim.y) - 1 - int(blockIdx.y) : int(blockIdx.y) - half);
   const int nk = min(q0 + 16, M), nch = (nk + 31) / 32;
   // Q fragments (rows past M read row M - 1: their outputs are not stored)
   uint4 qh[2], ql[2];
@@ -1047,9 +1051,9 @@ __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const flo
       const float bm = wave_max(fmaxf(fmaxf(s[h][0], s[h][1]), fmaxf(s[h][2], s[h][3])));
       mx[h] = fmaxf(mx[h], bm);
       const float nm = mx[h] == -INFINITY ? 0.f : mx[h];   // (only scores of -inf so far: weights 0)
-      const float al = expf(old[h] - nm);
+      const float al = exp_hw(old[h] - nm);
 #pragma unroll
-      for (int i = 0; i < kLd; ++i) s[h][i] = expf(s[h][i] - nm);
+      for (int i = 0; i < kLd; ++i) s[h][i] = exp_hw(s[h][i] - nm);
       ls[h] = ls[h] * al + ((s[h][0] + s[h][1]) + (s[h][2] + s[h][3]));
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[h][e] *= al;
@@ -1097,7 +1101,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const flo
     float num0 = 0.f, num1 = 0.f, den = 0.f;
 #pragma unroll
     for (int w = 0; w < kAttnWaves; ++w) {
-      const float a = expf(sm[w][h] - M);
+      const float a = exp_hw(sm[w][h] - M);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float2 v = *reinterpret_cast<const float2*>(so[w][r][h] + e);
