@@ -379,6 +379,13 @@ __device__ __forceinline__ void qkv_quad(f32x4 v, const float* rp, int col, int 
   }
 }
 
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+template <bool NT>
+__device__ __forceinline__ uint4 load_w(const uint16_t* p) {
+  const u32x4v* q = reinterpret_cast<const u32x4v*>(p);
+  return __builtin_bit_cast(uint4, NT ? __builtin_nontemporal_load(q) : *q);
+}
+
 // C = A W^T for many rows: a workgroup owns 16 RT rows x 16 CT columns over the whole of K, so it
 // streams 16 CT complete weight rows (contiguous in memory), every weight tile it loads serves
 // 16 RT rows, and it writes final outputs (no split-K partials).  The last column group may be
@@ -394,7 +401,10 @@ __device__ __forceinline__ void qkv_quad(f32x4 v, const float* rp, int col, int 
 // EPI: store the outputs, add them to the residual out (tile order; with an act plane also the
 // hi/lo tiles of scale * h and the row's partial sum of h^2 for the next RMSNorm), or finish them
 // in place of mx_swiglu_fin / mx_qkv_fin (the same arithmetic).
-template <int RT, int CT, int P, int NW, int AM, bool TW, int EPI>
+// Measured at 306M in the pass (one 16-row tile per workgroup and scalar epilogues before): gate/up of
+// 511 rows 31.8 -> 18.8 us, of 128 11.8 -> 10.2, of 5 7.2 -> 5.3; what bounds it is in rows_tile.
+// NT: the weights are read non-temporal (layers past kKeepBytes).
+template <int RT, int CT, int P, int NW, int AM, bool TW, int EPI, bool NT = false>
 __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
   static_assert(RT == 1 || (AM >= 1 && TW), "several row tiles per workgroup: tile-order operands");
   // the waves' partial tiles of one row tile, a lane's four outputs as one 16-byte piece (written and
@@ -458,7 +468,7 @@ __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
     const int ks = min(wv + NW * min(i, ns - 1), S - 1);
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)
-      w[p][ct] = *reinterpret_cast<const uint4*>(wr + min(ct, ctn - 1) * wtile + max(ks, 0) * wstep);
+      w[p][ct] = load_w<NT>(wr + min(ct, ctn - 1) * wtile + max(ks, 0) * wstep);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       a[p][rt] = *reinterpret_cast<const uint4*>(ar[rt] + max(ks, 0) * astep);
@@ -1150,7 +1160,6 @@ static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const f
 // mx_gemm's fragment loads of the row layout are 64 requests of 16 bytes each and bound it: 203 rows
 // of d 768 93 us, here 32.5; 24 rows of d 1024 33 us, here 15.8 (65 MB: 13 us at the card's
 // copy rate).  TOK: 32 and 64 where the rows fit, else 128 (LDS reads per MFMA fall with TOK).
-typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 template <int RB, int CB>
 struct LogitFrags {
   u32x4v w[RB], x[2][CB];
@@ -1285,6 +1294,7 @@ __global__ __launch_bounds__(256) void mx_logits(const uint16_t* X, int64_t plan
 __global__ __launch_bounds__(1024) void mx_argmax(const float* logits, int V, int ld, int32_t* out,
                                                   const int32_t* status, int nflags, float* copy) {
   __shared__ uint64_t red[16];
+  __shared__ int rflags[16];
   int flags = 0;
   for (int i = threadIdx.x; i < nflags; i += 1024) flags |= status[i];
   const float* lr = logits + int64_t(blockIdx.x) * ld;
@@ -1308,13 +1318,20 @@ __global__ __launch_bounds__(1024) void mx_argmax(const float* logits, int V, in
     const uint64_t w = __shfl_xor(best, o);
     best = w > best ? w : best;
   }
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
-  const int tok = __syncthreads_or(flags & 2), pos = __syncthreads_or(flags & 4);
+  flags = (__any(flags & 2) ? 2 : 0) | (__any(flags & 4) ? 4 : 0);
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = best;
+    rflags[threadIdx.x >> 6] = flags;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
     uint64_t b = red[0];
-    for (int i = 1; i < 16; ++i) b = red[i] > b ? red[i] : b;
+    for (int i = 1; i < 16; ++i) {
+      b = red[i] > b ? red[i] : b;
+      flags |= rflags[i];
+    }
     out[2 * blockIdx.x] = int32_t(0xffffffffu - uint32_t(b & 0xffffffffu));
-    out[2 * blockIdx.x + 1] = (tok ? 2 : 0) | (pos ? 4 : 0);
+    out[2 * blockIdx.x + 1] = flags;
   }
 }
 
@@ -1524,13 +1541,16 @@ static void launch_rows_packed(int ct, int grid, hipStream_t s, const GemmArgs& 
 // K steps in flight per wave: 4 while the tile leaves the registers for it (single residual tiles of 4
 // waves: 8, all of a 1024-wide projection; more gained nothing elsewhere)
 template <int AM, int EPI, int I = 0>
-static void launch_rows_tiles(const RowsTile& t, int grid, hipStream_t s, const GemmArgs& g) {
+static void launch_rows_tiles(const RowsTile& t, int grid, hipStream_t s, const GemmArgs& g, bool nt) {
   constexpr RowsTile k = kRowsTiles[I];
   if (t.rt == k.rt && t.ct == k.ct && t.nw == k.nw) {
     constexpr int P = k.rt * k.ct == 1 && k.nw == 4 && EPI == kEpiResid ? 8 : k.rt == 1 && k.ct <= 4 ? 4 : (k.rt * k.ct <= 6 ? 3 : 2);
-    hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI>), dim3(grid), dim3(64 * k.nw), 0, s, g);
+    if (nt)
+      hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI, true>), dim3(grid), dim3(64 * k.nw), 0, s, g);
+    else
+      hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI>), dim3(grid), dim3(64 * k.nw), 0, s, g);
   } else if constexpr (I + 1 < int(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))) {
-    launch_rows_tiles<AM, EPI, I + 1>(t, grid, s, g);
+    launch_rows_tiles<AM, EPI, I + 1>(t, grid, s, g, nt);
   }
 }
 
@@ -1551,7 +1571,8 @@ static void launch_splitk(int bm, dim3 grid, hipStream_t s, const GemmArgs& g) {
 // bitwise the same either way.
 static hipError_t gemm(const uint16_t* A, int64_t a_plane, int lda, const uint16_t* W, bool tw, int M, int N, int K,
                        float* out, int ldo, int splits, hipStream_t s, bool rows_ok = true, int epi = kEpiStore,
-                       const EpiArgs* ea = nullptr, const float* ssq = nullptr, int nssq = 0) {
+                       const EpiArgs* ea = nullptr, const float* ssq = nullptr, int nssq = 0,
+                       bool nt = false) {
   GemmArgs g{A, a_plane, W, out, M, N, K, lda, ldo, splits, ea ? *ea : EpiArgs{}, ssq, nssq};
   const int am = ssq ? 2 : (lda == 0 ? 1 : 0);
   if ((epi != kEpiStore) != tw || (epi != kEpiStore && (!ea || am == 0 || splits != 1)))
@@ -1561,9 +1582,9 @@ static hipError_t gemm(const uint16_t* A, int64_t a_plane, int lda, const uint16
   if (tw) {
     const RowsTile t = rows_tile(M, N, K, epi == kEpiResid ? kMaxGroups : 0);
     const int grid = ((T + t.rt - 1) / t.rt) * ((N / 16 + t.ct - 1) / t.ct);
-    if (am == 2 && epi == kEpiQkv) launch_rows_tiles<2, kEpiQkv>(t, grid, s, g);
-    else if (am == 2 && epi == kEpiSwiglu) launch_rows_tiles<2, kEpiSwiglu>(t, grid, s, g);
-    else if (am == 1 && epi == kEpiResid) launch_rows_tiles<1, kEpiResid>(t, grid, s, g);
+    if (am == 2 && epi == kEpiQkv) launch_rows_tiles<2, kEpiQkv>(t, grid, s, g, nt);
+    else if (am == 2 && epi == kEpiSwiglu) launch_rows_tiles<2, kEpiSwiglu>(t, grid, s, g, nt);
+    else if (am == 1 && epi == kEpiResid) launch_rows_tiles<1, kEpiResid>(t, grid, s, g, nt);
     else return hipErrorInvalidValue;
     return hipGetLastError();
   }
@@ -1614,6 +1635,17 @@ static int64_t first_norm_scales(const msd_config* c) {
   const int64_t d = c->d_model, ff = c->d_ff, nqkv = int64_t(c->n_heads + 2 * c->n_kv_heads) * kDh;
   return nqkv * d + d * d + 2 * ff * d + d * ff;
 }
+
+// Weights that do not fit the 256 MB last-level cache (tile copies past kCacheBytes) are split: the first
+// layers, up to kKeepBytes, are read with the default policy and stay there from one pass to the
+// next, the others non-temporal, so they stream past. Measured at 306M (541 MB; none / 90 / 130 / 160
+// MiB kept): verification of 5 tokens 646 / 604 / 595 / 593 us, prefill of 16 686 / 643 / 632 / 629, of
+// 64 722 / 685 / 676 / 675, of 128 849 / 834 / 823 / 817. Past 128 rows it loses (200 rows 1095 / 1170 /
+// 1149 / 1141: a weight tile then serves many row tiles' workgroups, and its lines leave the L2 before
+// the last has read them), and a batched step's own K/V rows (127 MB for 24 sequences) need the
+// cache (735 / 729 / 737 / 739): both keep the default policy throughout.
+constexpr int64_t kKeepBytes = int64_t(150) << 20, kCacheBytes = int64_t(224) << 20;
+constexpr int kStreamRows = 128;
 
 // The layer stack over M rows whose residual stream is already in h; leaves the last
 // projection's partials pending (returned split count).
@@ -1668,7 +1700,10 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
       // adding to h and writing the next layer's RMSNorm1 input planes.
       const uint16_t* Tl = wt.tiles + int64_t(l) * tile_layer_elems(cfg);
       const bool last = l + 1 == cfg->n_layers;
-      if ((err = gemm(xn, pd, 0, Tl, true, M, nqkv, d, nullptr, 0, 1, s, true, kEpiQkv, &eq, ssq, l == 0 ? 1 : cg_d)) !=
+      const int64_t bytes = 2 * tile_layer_elems(cfg);
+      const bool nt = M <= kStreamRows && !rows.batched && cfg->n_layers * bytes > kCacheBytes && (l + 1) * bytes > kKeepBytes;
+      if ((err = gemm(xn, pd, 0, Tl, true, M, nqkv, d, nullptr, 0, 1, s, true, kEpiQkv, &eq, ssq, l == 0 ? 1 : cg_d,
+                      nt)) !=
           hipSuccess)
         break;
       if (prefill)
@@ -1680,17 +1715,20 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
       en.act_plane = pd;
       en.ssq = ssq;
       en.xscale = Tl + toff_sc + d;
-      if ((err = gemm(att, pd, 0, Tl + toff_o, true, M, d, d, h, d, 1, s, true, kEpiResid, &en)) != hipSuccess)
+      if ((err = gemm(att, pd, 0, Tl + toff_o, true, M, d, d, h, d, 1, s, true, kEpiResid, &en, nullptr, 0,
+                      nt)) != hipSuccess)
         break;
       EpiArgs eg{};
       eg.act = act;
       eg.act_plane = pf;
-      if ((err = gemm(xn, pd, 0, Tl + toff_gu, true, M, 2 * ff, d, nullptr, 0, 1, s, true, kEpiSwiglu, &eg, ssq, cg_o)) !=
+      if ((err = gemm(xn, pd, 0, Tl + toff_gu, true, M, 2 * ff, d, nullptr, 0, 1, s, true, kEpiSwiglu, &eg, ssq, cg_o,
+                      nt)) !=
           hipSuccess)
         break;
       if (last) en.act = nullptr;   // (the final norm reads h)
       else en.xscale = Tl + tile_layer_elems(cfg) + toff_sc;   // the next layer's RMSNorm1
-      if ((err = gemm(act, pf, 0, Tl + toff_dn, true, M, d, ff, h, d, 1, s, true, kEpiResid, &en)) != hipSuccess)
+      if ((err = gemm(act, pf, 0, Tl + toff_dn, true, M, d, ff, h, d, 1, s, true, kEpiResid, &en, nullptr, 0,
+                      nt)) != hipSuccess)
         break;
       continue;
     }
