@@ -6,6 +6,7 @@
  *                         logsumexp(h W^T) - (h W^T)[target], without storing the logits
  *   msd_xent_backward  <- model.py:320-361 _fused_ce_bwd (the custom_vjp backward, :364):
  *                         grad_h and grad_weight of that loss times the incoming gradient g
+ *   msd_xent_targets   (no counterpart: the int32 targets both take, converted and checked)
  *   msd_xent_workspace_bytes
  *                      <- the chunk buffers of the reference's loops (model.py:293-301, 344-353)
  *

@@ -66,8 +66,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kStatusTarget = 4;  // a target id outside [0, V) (replaced by 0)
 
-__device__ __forceinline__ bf16x8 as_bf(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
-
 // round to nearest even (finite inputs; NaN stays NaN)
 __device__ __forceinline__ uint16_t f2bf(float x) {
   const uint32_t u = __float_as_uint(x);
