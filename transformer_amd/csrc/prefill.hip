@@ -52,6 +52,7 @@
 #include <vector>
 
 #include "../../include/msdecode.h"
+#include "arith.h"
 #include "batched.h"
 #include "internal.h"
 
@@ -316,13 +317,8 @@ __global__ __launch_bounds__(256) void mx_gemm(GemmArgs g) {
       }
 }
 
-// exp(x) by the hardware base-2 exponential (x log2(e) rounded once: |x| 2^-24 relative)
-__device__ __forceinline__ float exp_hw(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
-
-// SwiGLU of a gate/up pair (packed rows 2f, 2f + 1; model.py:159).
-__device__ __forceinline__ float swiglu(float g, float u) {
-  return (g * __builtin_amdgcn_rcpf(1.f + exp_hw(-g))) * u;
-}
+using msdc::quotient;
+using msdc::swiglu;   // of a gate/up pair: packed rows 2f, 2f + 1
 
 // Four outputs of the packed q/k/v rows col .. col + 3 (col a multiple of 4) of row `row`, whose position
 // has the RoPE row rp: q and k pairs are rotated (dims i, i + 32; model.py:110-117), v is stored
@@ -410,7 +406,7 @@ __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
   // the waves' partial tiles of one row tile, a lane's four outputs as one 16-byte piece (written and
   // read across lanes contiguously); two buffers, so one barrier per row tile suffices
   __shared__ f32x4 red[RT > 1 ? 2 : 1][NW][CT][64];
-  __shared__ float rrms[16 * RT];       // AM 2: each row's 1 / rms
+  __shared__ float rms[2][16 * RT];     // AM 2: each row's rms and its reciprocal
   __shared__ float hs[RT][NW][16];      // kEpiResid: each wave's part of the rows' sums of h^2
   // wave-uniform wave index: the step count and its loop stay scalar (a per-lane loop would copy
   // the accumulators out of and back into the AGPRs around every step)
@@ -531,7 +527,11 @@ __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
       for (int j = 0; j < kSq; ++j) sum += int(threadIdx.x & 15) + 16 * j < g.nssq ? sq[q][j] : 0.f;
       sum = sum16_lanes(sum);
       const int row = int(threadIdx.x >> 4) + 4 * NW * q;
-      if ((threadIdx.x & 15) == 0 && row < 16 * RT) rrms[row] = 1.f / sqrtf(sum / float(g.K) + 1e-5f);
+      if ((threadIdx.x & 15) == 0 && row < 16 * RT) {
+        const float r = sqrtf(sum / float(g.K) + 1e-5f);
+        rms[0][row] = r;
+        rms[1][row] = 1.f / r;
+      }
     }
   }
 #pragma unroll
@@ -559,7 +559,11 @@ __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
       f32x4 v = rd[0][ct][lane];
 #pragma unroll
       for (int w2 = 1; w2 < NW; ++w2) v += rd[w2][ct][lane];
-      if constexpr (AM == 2) v *= rrms[16 * rt + orow];
+      if constexpr (AM == 2) {
+        const float r = rms[0][16 * rt + orow], rr = rms[1][16 * rt + orow];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = quotient(v[e], r, rr);
+      }
       const int col = n0 + 16 * ct + ocol;
       if (!live) continue;
       if constexpr (EPI == kEpiStore) {
@@ -881,8 +885,8 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
       const float v0 = (j0 <= i && j0 < M) ? s[0][r] * 0.125f : -INFINITY;
       const float v1 = (j1 <= i && j1 < M) ? s[1][r] * 0.125f : -INFINITY;
       const float mn = fmaxf(m[r], row16_max(fmaxf(v0, v1)));
-      const float p0 = mn == -INFINITY ? 0.f : exp_hw(v0 - mn), p1 = mn == -INFINITY ? 0.f : exp_hw(v1 - mn);
-      const float alpha = m[r] == -INFINITY ? 0.f : exp_hw(m[r] - mn);
+      const float p0 = mn == -INFINITY ? 0.f : expf(v0 - mn), p1 = mn == -INFINITY ? 0.f : expf(v1 - mn);
+      const float alpha = m[r] == -INFINITY ? 0.f : expf(m[r] - mn);
       l[r] = l[r] * alpha + row16_sum(p0 + p1);
       m[r] = mn;
 #pragma unroll
@@ -922,7 +926,7 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
   float L = 0.f, O[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    const float wt = sm[w][qi] == -INFINITY ? 0.f : exp_hw(sm[w][qi] - mx);
+    const float wt = sm[w][qi] == -INFINITY ? 0.f : expf(sm[w][qi] - mx);
     L += sl[w][qi] * wt;
 #pragma unroll
     for (int e = 0; e < 4; ++e) O[e] += so[w][qi][d4 + e] * wt;
@@ -1061,9 +1065,9 @@ __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const flo
       const float bm = wave_max(fmaxf(fmaxf(s[h][0], s[h][1]), fmaxf(s[h][2], s[h][3])));
       mx[h] = fmaxf(mx[h], bm);
       const float nm = mx[h] == -INFINITY ? 0.f : mx[h];   // (only scores of -inf so far: weights 0)
-      const float al = exp_hw(old[h] - nm);
+      const float al = expf(old[h] - nm);
 #pragma unroll
-      for (int i = 0; i < kLd; ++i) s[h][i] = exp_hw(s[h][i] - nm);
+      for (int i = 0; i < kLd; ++i) s[h][i] = expf(s[h][i] - nm);
       ls[h] = ls[h] * al + ((s[h][0] + s[h][1]) + (s[h][2] + s[h][3]));
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[h][e] *= al;
@@ -1111,7 +1115,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const flo
     float num0 = 0.f, num1 = 0.f, den = 0.f;
 #pragma unroll
     for (int w = 0; w < kAttnWaves; ++w) {
-      const float a = exp_hw(sm[w][h] - M);
+      const float a = expf(sm[w][h] - M);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float2 v = *reinterpret_cast<const float2*>(so[w][r][h] + e);
