@@ -214,7 +214,7 @@ int32_t msd_sample_token_noalloc(const float* logits, int32_t vocab, double temp
                                  double rep_penalty, uint8_t* seen, const double* uniform,
                                  int32_t* token_out, float* probs_out, int32_t* kept_out, void* stream);
 
-/* Bytes of device workspace msd_prefill needs for a prompt of n_tokens tokens. */
+/* Bytes of device workspace msd_prefill needs for a prompt of up to n_tokens tokens. */
 int64_t msd_prefill_workspace_bytes(const msd_config* cfg, int32_t n_tokens);
 
 /* Bytes of the tile copy of the layer weights (the QKV, O, gate/up and down matrices and the two
@@ -264,7 +264,7 @@ int32_t msd_prefill(const msd_config* cfg, const void* token_emb, const void* ou
  * launch-mode switch of this library. */
 int32_t msd_set_launch_graphs(int32_t enabled);
 
-/* Bytes of device workspace msd_verify needs for n_tokens rows. */
+/* Bytes of device workspace msd_verify needs for up to n_tokens rows. */
 int64_t msd_verify_workspace_bytes(const msd_config* cfg, int32_t n_tokens);
 
 /* Speculative-decode verification: the target model's forward pass over tokens[0..n_tokens)
@@ -300,7 +300,7 @@ int32_t msd_prefill_paged(const msd_config* cfg, const void* token_emb, const vo
                           int32_t max_pages, void* kv_pool, int32_t pool_pages, void* workspace,
                           float* logits_last, int32_t* next_token, void* stream);
 
-/* Bytes of device workspace msd_batch_decode_step needs for `batch` sequences.  The workspace
+/* Bytes of device workspace msd_batch_decode_step needs for up to `batch` sequences.  The workspace
  * must be zero-filled before its first step and then kept for the steps of this batch decoder
  * (it holds the persistent step's epoch and barrier flags); one step may be in flight per
  * workspace.  Any device memory works; for the persistent step (batch <= 8 on a config with

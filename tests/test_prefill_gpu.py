@@ -133,6 +133,26 @@ def test_tile_choices_match_the_packed_rows(wide, T):
     assert float((a - b).norm()) <= 1e-3 * float(b.norm())
 
 
+@pytest.mark.parametrize("cap,T", [(48, 47), (65, 64), (129, 128), (300, 256)])
+@pytest.mark.parametrize("tiles", [True, False], ids=["tiles", "rows"])
+def test_shorter_prompts_stay_inside_a_larger_workspace(wide, cap, T, tiles):
+    """A prompt shorter than max_tokens splits K more: its partials, flags and page rows stay inside the
+    workspace sized for max_tokens, and the pass gives the bits of one sized for the prompt."""
+    toks = make_prompt(T, WIDE["vocab_size"], seed=T)
+    la, _, out, kv = _run(wide, WIDE, toks, tiles=tiles)
+    pf = Prefiller(wide, WIDE, max_tokens=cap, tiles=tiles)
+    n = pf.workspace.numel()
+    guarded = torch.full((2 * n,), 0x5A, dtype=torch.uint8, device="cuda")
+    pf.workspace = guarded[:n]
+    kv2 = new_kv_packed(WIDE).fill_(SENTINEL)
+    la2 = torch.empty((T, WIDE["vocab_size"]), dtype=torch.float32, device="cuda")
+    out2 = pf.launch(toks, kv2, logits_all=la2)
+    torch.cuda.synchronize()
+    assert bool((guarded[n:] == 0x5A).all()), "written past the workspace"
+    assert np.array_equal(la2.cpu().numpy(), la) and np.array_equal(out2.cpu().numpy(), out)
+    assert torch.equal(kv2, kv)
+
+
 def test_306m_prefill_128_matches_oracle(m306):
     """The prefill of a 128-token prompt on the 306M configuration."""
     params, w = m306

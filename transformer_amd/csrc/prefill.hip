@@ -1500,10 +1500,23 @@ static size_t part_floats(const msd_config* c, int M) {
   return mx * M;
 }
 
+// The largest part_floats over passes of 1..M rows: a pass of fewer rows may split K more and need more
+// (306M: 128 rows 9.4 MB of partials, 129 rows 4.2).  The split counts change with the number of
+// 16-row tiles and at 48 rows only, and are 1 for every N past kRowsPerPass rows, so the last two row
+// counts of each 16 cover them all.
+static size_t part_floats_upto(const msd_config* c, int M) {
+  constexpr int kRowsPerPass = 128 * 256;   // a 128-row tile per CU
+  size_t mx = part_floats(c, M);
+  for (int m = 16; m < M + 16 && m <= kRowsPerPass; m += 16)
+    for (int q : {m - 1, m}) mx = std::max(mx, part_floats(c, std::min(q, M)));
+  return mx;
+}
+
 static int pad16(int M) { return (M + 15) & ~15; }
 static int pad32(int M) { return (M + 31) & ~31; }
 
-static Layout layout(const msd_config* c, int M) {
+// part: floats of the split-K partials
+static Layout layout(const msd_config* c, int M, size_t part) {
   const int d = c->d_model, ff = c->d_ff, nqkv = (c->n_heads + 2 * c->n_kv_heads) * kDh;
   Layout L;
   size_t o = 0;
@@ -1515,12 +1528,18 @@ static Layout layout(const msd_config* c, int M) {
   L.kvp = o;    o += al256(size_t(pad32(M)) * c->n_kv_heads * kDh * 2 * 4);   // prefill: K/V operand planes
   L.att = o;    o += al256(size_t(pad16(M)) * d * 2 * 2);
   L.act = o;    o += al256(size_t(pad16(M)) * ff * 2 * 2);
-  L.part = o;   o += al256(part_floats(c, M) * 4);
+  L.part = o;   o += al256(part * 4);
   L.status = o; o += al256(size_t(M) * 2 * 4);   // flags: each row's token, then each row's position
   L.rowpos = o; o += al256(size_t(M) * 4);
   L.pages = o;  o += al256(size_t(M) * ((c->context_len + kPage - 1) / kPage) * 4);
   L.bytes = o;
   return L;
+}
+static Layout layout(const msd_config* c, int M) { return layout(c, M, part_floats(c, M)); }
+
+// Bytes that hold any pass of 1..M rows (every other region grows with the rows).
+static int64_t workspace_bytes(const msd_config* c, int M) {
+  return int64_t(layout(c, M, part_floats_upto(c, M)).bytes);
 }
 
 static bool mx_config_ok(const msd_config* c) {
@@ -1863,7 +1882,7 @@ using namespace mpf;
 extern "C" int64_t msd_prefill_workspace_bytes(const msd_config* cfg, int32_t n_tokens) {
   if (!mx_config_ok(cfg)) return MSD_E_CONFIG;
   if (n_tokens <= 0 || n_tokens > cfg->context_len) return MSD_E_ARG;
-  return int64_t(layout(cfg, n_tokens).bytes);
+  return workspace_bytes(cfg, n_tokens);
 }
 
 // The forward pass over tokens[0..n_tokens) at positions start..start+n_tokens-1.  With
@@ -2013,7 +2032,7 @@ static int64_t batch_region(const msd_config* cfg) { return (mbd::region_bytes(c
 extern "C" int64_t msd_batch_workspace_bytes(const msd_config* cfg, int32_t batch) {
   if (!mx_config_ok(cfg)) return MSD_E_CONFIG;
   if (batch <= 0 || batch > kMaxRows) return MSD_E_ARG;
-  return batch_region(cfg) + int64_t(layout(cfg, batch).bytes);
+  return batch_region(cfg) + workspace_bytes(cfg, batch);
 }
 
 extern "C" int32_t msd_batch_decode_step(const msd_config* cfg, const void* token_emb, const void* output_proj,
