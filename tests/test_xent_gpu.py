@@ -110,6 +110,69 @@ def test_deterministic_and_3d_wrapper():
     assert np.array_equal(gw.float().cpu().numpy(), a[2])
 
 
+def _loss_and_grads(x, check):
+    h, w, t = x
+    loss = fused_cross_entropy(h, w, t, 512, check_targets=check)
+    return (loss.detach(), *torch.autograd.grad(loss, (h, w)))
+
+
+def _several_inputs(n):
+    out = []
+    for i in range(n):
+        h, w, t = _inputs(200, 9000, 256, seed=20 + i)
+        out.append((h.cuda().requires_grad_(), w.cuda().requires_grad_(), t.cuda()))
+    return out
+
+
+@pytest.mark.parametrize("check", [True, False])
+def test_calls_on_several_streams_do_not_share_scratch(check):
+    """Losses of one shape issued on two streams, nothing waited for between them: each has the bits of
+    the same call alone."""
+    xs = _several_inputs(2)
+    alone = [_loss_and_grads(x, check) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    got = [[] for _ in xs]
+    for _ in range(8):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i].append(_loss_and_grads(xs[i], check))
+    torch.cuda.synchronize()
+    for i, runs in enumerate(got):
+        for r in runs:
+            assert all(torch.equal(a, b) for a, b in zip(r, alone[i]))
+
+
+def test_calls_from_several_threads_do_not_share_scratch():
+    """The same from two host threads on one stream, whose launches interleave."""
+    import threading
+    xs = _several_inputs(2)
+    alone = [_loss_and_grads(x, False) for x in xs]
+    torch.cuda.synchronize()
+    got, errors = [[] for _ in xs], []
+
+    def work(i):
+        try:
+            for _ in range(8):
+                got[i].append(_loss_and_grads(xs[i], False))
+        except Exception as e:   # reported by the test's own thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(xs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i, runs in enumerate(got):
+        assert len(runs) == 8
+        for r in runs:
+            assert all(torch.equal(a, b) for a, b in zip(r, alone[i]))
+
+
 def test_bad_targets_and_arguments():
     h, w, t = _inputs(64, 500, 128, seed=7)
     t[3] = 500

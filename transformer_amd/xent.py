@@ -22,6 +22,7 @@ block is rounded to bf16 before its two products (the reference keeps f32; both 
 gradients).
 """
 import ctypes
+import functools
 
 import torch
 
@@ -30,20 +31,15 @@ from . import _lib
 STATUS_BAD_TARGET = 4
 
 
-class _Workspace:
-    """Device workspace per (device, N, V, d, chunk), kept for reuse."""
-    cache = {}
+@functools.lru_cache(maxsize=64)
+def _workspace_bytes(n, V, d, chunk):
+    return _lib.check(_lib.lib().msd_xent_workspace_bytes(n, V, d, chunk), "msd_xent_workspace_bytes")
 
-    @classmethod
-    def get(cls, device, n, V, d, chunk):
-        key = (str(device), n, V, d, chunk)
-        ws = cls.cache.get(key)
-        if ws is None:
-            nbytes = _lib.check(_lib.lib().msd_xent_workspace_bytes(n, V, d, chunk), "msd_xent_workspace_bytes")
-            if len(cls.cache) >= 4:
-                cls.cache.pop(next(iter(cls.cache)))
-            ws = cls.cache[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        return ws
+
+def _workspace(device, n, V, d, chunk):
+    """The device workspace of one call, from torch's caching allocator: calls on several streams or
+    threads never share one, and the block is used again in stream order once the call has returned."""
+    return torch.empty(_workspace_bytes(n, V, d, chunk), dtype=torch.uint8, device=device)
 
 
 def _check_inputs(h, weight, targets):
@@ -69,7 +65,7 @@ class FusedCrossEntropy(torch.autograd.Function):
         N, d = h.shape
         V = weight.shape[0]
         chunk = int(chunk_size)
-        ws = _Workspace.get(h.device, N, V, d, chunk)
+        ws = _workspace(h.device, N, V, d, chunk)
         loss = torch.empty((), dtype=torch.float32, device=h.device)
         lse = torch.empty(N, dtype=torch.float32, device=h.device)
         # int32 targets and the status word behind them
@@ -100,7 +96,7 @@ class FusedCrossEntropy(torch.autograd.Function):
         h, weight, tg, lse = ctx.saved_tensors
         N, d = h.shape
         V = weight.shape[0]
-        ws = _Workspace.get(h.device, N, V, d, ctx.chunk)
+        ws = _workspace(h.device, N, V, d, ctx.chunk)
         gl = g.detach().to(torch.float32).reshape(1).contiguous()
         grad_h = torch.empty_like(h)
         grad_w = torch.empty_like(weight)
