@@ -35,8 +35,8 @@ extern "C" {
 int64_t msd_xent_workspace_bytes(int32_t n_rows, int32_t vocab, int32_t d_model, int32_t chunk);
 
 /* Targets for the calls below: int32 copies (out, n_rows) of n_rows int32 (bytes_each 4) or int64
- * (bytes_each 8, low words) device targets, and in *status (written, not accumulated) 4 if any is
- * outside [0, vocab), else 0.  For callers that hold int64 targets or check them before the forward. */
+ * (bytes_each 8) device targets, an id outside [0, vocab) as -1 (used as 0 by the calls below), and in
+ * *status (written, not accumulated) 4 if there is any, else 0.  For callers that hold int64 targets or check them before the forward. */
 int32_t msd_xent_targets(const void* targets, int32_t bytes_each, int32_t n_rows, int32_t vocab, int32_t* out,
                          int32_t* status, void* stream);
 

@@ -175,9 +175,14 @@ def test_calls_from_several_threads_do_not_share_scratch():
 
 def test_bad_targets_and_arguments():
     h, w, t = _inputs(64, 500, 128, seed=7)
-    t[3] = 500
-    with pytest.raises(ValueError, match="target"):
-        fused_cross_entropy(h.cuda(), w.cuda(), t.cuda(), 256)
+    for bad in (500, -1, 2 ** 32 + 5, -2 ** 32 + 5):   # the last two are valid in their low 32 bits
+        t[3] = bad
+        with pytest.raises(ValueError, match="target"):
+            fused_cross_entropy(h.cuda(), w.cuda(), t.cuda(), 256)
+        unchecked = fused_cross_entropy(h.cuda(), w.cuda(), t.cuda(), 256, check_targets=False)
+        t[3] = 0
+        assert torch.equal(unchecked, fused_cross_entropy(h.cuda(), w.cuda(), t.cuda(), 256)), "not used as 0"
+    assert torch.equal(unchecked, fused_cross_entropy(h.cuda(), w.cuda(), t.cuda().to(torch.int16), 256))
     with pytest.raises(ValueError):
         fused_cross_entropy(h.cuda().float(), w.cuda(), t.cuda(), 256)      # f32 h
     with pytest.raises(ValueError):

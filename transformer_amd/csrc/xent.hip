@@ -620,16 +620,17 @@ __global__ __launch_bounds__(256) void xent_sum_parts(const float* part, int spl
       make_uint2(f2bf(s.x) | (uint32_t(f2bf(s.y)) << 16), f2bf(s.z) | (uint32_t(f2bf(s.w)) << 16));
 }
 
-// Targets as int32 (from int32, or the low words of int64) and, in status[0], whether any is outside
-// [0, V).  One workgroup: it needs no cleared status word and is done long before the logits GEMM,
+// Targets as int32 and, in status[0], whether any is outside [0, V): such an id, compared at its own width,
+// becomes -1, which the other kernels take as 0.  One workgroup: it needs no cleared status word and is done long before the logits GEMM,
 // so a caller that checks waits for this kernel only.
 template <typename I>
 __global__ __launch_bounds__(1024) void xent_targets(const I* targets, int n, int V, int32_t* out, int32_t* status) {
   bool bad = false;
   for (int i = threadIdx.x; i < n; i += 1024) {
-    const int32_t t = int32_t(targets[i]);
-    out[i] = t;
-    bad |= t < 0 || t >= V;
+    const I t = targets[i];
+    const bool in = t >= 0 && t < V;
+    out[i] = in ? int32_t(t) : -1;
+    bad |= !in;
   }
   bad = __syncthreads_or(bad);
   if (threadIdx.x == 0) status[0] = bad ? kStatusTarget : 0;

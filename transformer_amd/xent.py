@@ -70,7 +70,7 @@ class FusedCrossEntropy(torch.autograd.Function):
         lse = torch.empty(N, dtype=torch.float32, device=h.device)
         # int32 targets and the status word behind them
         tg = torch.empty(N + 1, dtype=torch.int32, device=h.device)
-        raw = (targets if targets.dtype in (torch.int32, torch.int64) else targets.to(torch.int32)).contiguous()
+        raw = (targets if targets.dtype in (torch.int32, torch.int64) else targets.to(torch.int64)).contiguous()
         s = torch.cuda.current_stream(h.device)
         stream = ctypes.c_void_p(s.cuda_stream)
         status = tg.data_ptr() + 4 * N
