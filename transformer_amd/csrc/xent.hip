@@ -705,33 +705,49 @@ int rup(int x, int m) { return (x + m - 1) / m * m; }
 struct Plan {
   int Np;          // tokens padded to 256
   int C;           // vocabulary ids per chunk (a multiple of 256)
+  bool big_f;      // 256-tiles for the forward's S^T (the whole vocabulary)
   bool big_s, big_w, big_h;   // 256-tiles for S^T, grad_W, grad_h
   int splits, k_split;        // grad_h: K splits of a chunk, K per split (a multiple of 64)
 };
-constexpr double kFill = 0.8;
-constexpr int64_t kBlockBytes = int64_t(256) << 20;
+constexpr double kFill = 0.8, kSplits = 0.75;
+constexpr int64_t kBlockBytes = int64_t(256) << 20, kRoomBytes = int64_t(64) << 20;
 
 int cdiv(int x, int m) { return (x + m - 1) / m; }
 
 Plan plan(int n, int V, int d, int chunk) {
   Plan p;
   p.Np = rup(n, 256);
-  const int Vp = rup(V, 256);
-  // The caller's chunk is raised to a block of kBlockBytes (of 288 GB): few chunks are what fills
-  // the chip (N 509: 8 chunks 1027 us, one 249; N 4096, V 32000: blocks of 128 MiB 1240 us, 256 1149).
-  const int fit = int(std::min<int64_t>(kBlockBytes / (2 * int64_t(p.Np)) / 256 * 256, Vp));
-  const int c = std::max(std::min(rup(std::max(chunk, 1), 256), Vp), fit);
-  p.C = rup(cdiv(Vp, cdiv(Vp, c)), 256);   // chunks of equal size
+  const int Vp = rup(V, 256), c0 = std::min(rup(std::max(chunk, 1), 256), Vp);
   auto fills = [](int m, int n, int tiles) {   // 256-tiles of m x n outputs on a multiple of 256 CUs
     return double(m) * n >= kFill * 65536.0 * 256 * cdiv(tiles, 256);
   };
   const int t256 = cdiv(n, 256) * cdiv(d, 256);
-  p.big_s = fills(p.C, n, p.C / 256 * cdiv(n, 256));
-  p.big_w = fills(p.C, d, p.C / 256 * cdiv(d, 256));
   // (grad_h's tiles are split over K until they fill the chip)
   p.big_h = t256 >= 32 && double(n) * d >= kFill * 65536.0 * t256;
   const int tiles = p.big_h ? t256 : cdiv(n, 128) * (d / 128);
-  const int want = std::max(1, std::min((p.big_h ? 256 : 512) / tiles, p.C / 512));
+  p.big_f = fills(Vp, n, Vp / 256 * cdiv(n, 256));
+  // Few chunks are what fills the chip (N 509, V 32000: eight chunks 1027 us, one 249), but the chunk is
+  // how a caller bounds the memory.  So the vocabulary is cut into as few equal chunks as keep the block
+  // within kBlockBytes (or the caller's own block), and the block with grad_h's partials within `room`:
+  // eight of the caller's blocks (fewer under 1024 ids, two at 256, the smallest) and the size of W, h
+  // and an f32 grad_h, of which W^T, h^T and one grad_h were once held; kRoomBytes in any case.
+  // kSplits of the splits that fill the chip are enough.
+  const int64_t block = 2 * int64_t(p.Np), part = 4 * int64_t(n) * d;
+  const int64_t room =
+      std::max(kRoomBytes, std::min(8, c0 / 128) * block * c0 + 2 * (int64_t(Vp) + p.Np) * d + 4 * int64_t(p.Np) * d -
+                               (p.big_f ? 0 : 8 * int64_t(Vp / 256) * p.Np));   // (more partials of the forward)
+  const int most = std::max<int>(c0, int(std::min<int64_t>(kBlockBytes / block / 256 * 256, Vp)));
+  int want = 1;
+  for (int k = cdiv(Vp, most);; ++k) {
+    p.C = rup(cdiv(Vp, k), 256);
+    want = std::max(1, std::min((p.big_h ? 256 : 512) / tiles, p.C / 512));
+    const int64_t got = std::max<int64_t>((room - block * p.C) / part, 0);
+    const bool enough = double(got) >= kSplits * want;
+    want = int(std::max<int64_t>(std::min<int64_t>(want, got), 1));
+    if (enough || p.C <= c0) break;
+  }
+  p.big_s = fills(p.C, n, p.C / 256 * cdiv(n, 256));
+  p.big_w = fills(p.C, d, p.C / 256 * cdiv(d, 256));
   p.k_split = rup(cdiv(p.C, want), 64);
   p.splits = cdiv(p.C, p.k_split);
   return p;
@@ -744,7 +760,7 @@ struct Layout {
 Layout layout(int n, int V, int d, const Plan& p) {
   Layout L;
   int64_t o = 0;
-  L.part = o;    o += al256(int64_t(rup(V, 256) / 128) * p.Np * 8);
+  L.part = o;    o += al256(int64_t(rup(V, 256) / (p.big_f ? 256 : 128)) * p.Np * 8);
   L.tgt = o;     o += al256(int64_t(p.Np) * 4);
   L.lrow = o;    o += al256(int64_t(p.Np) * 4);
   L.P = o;       o += al256(int64_t(p.Np) * p.C * 2);
@@ -784,6 +800,17 @@ extern "C" int64_t msd_xent_workspace_bytes(int32_t n_rows, int32_t vocab, int32
   return layout(n_rows, vocab, d_model, plan(n_rows, vocab, d_model, chunk)).bytes;
 }
 
+extern "C" int32_t msd_xent_plan(int32_t n_rows, int32_t vocab, int32_t d_model, int32_t chunk, int32_t* out) {
+  if (!out) return MSD_E_ARG;
+  if (!shape_ok(n_rows, vocab, d_model)) return MSD_E_CONFIG;
+  const Plan p = plan(n_rows, vocab, d_model, chunk);
+  const int chunks = cdiv(vocab, p.C), last = vocab - (chunks - 1) * p.C;
+  const int32_t v[8] = {p.C, chunks, p.big_f ? 256 : 128, p.big_s ? 256 : 128, p.big_w ? 256 : 128, p.big_h ? 256 : 128,
+                        cdiv(rup(std::min(p.C, vocab), 64), p.k_split), cdiv(rup(last, 64), p.k_split)};
+  std::copy(v, v + 8, out);
+  return MSD_OK;
+}
+
 extern "C" int32_t msd_xent_targets(const void* targets, int32_t bytes_each, int32_t n_rows, int32_t vocab, int32_t* out,
                                     int32_t* status, void* stream) {
   if (n_rows < 1 || vocab < 1) return MSD_E_CONFIG;
@@ -804,7 +831,7 @@ extern "C" int32_t msd_xent_forward(const void* h, const void* weight, const int
   if (!shape_ok(n_rows, vocab, d_model)) return MSD_E_CONFIG;
   if (!h || !weight || !targets || !workspace || !loss || !lse || !status) return MSD_E_ARG;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const Plan p = plan(n_rows, vocab, d_model, vocab);   // (its prefix of the workspace is the same for every chunk)
+  const Plan p = plan(n_rows, vocab, d_model, vocab);   // (what it takes of it is the same for every chunk)
   const Layout L = layout(n_rows, vocab, d_model, p);
   char* ws = static_cast<char*>(workspace);
   GemmArgs g{};
@@ -824,10 +851,10 @@ extern "C" int32_t msd_xent_forward(const void* h, const void* weight, const int
   g.part = reinterpret_cast<float*>(ws + L.part);
   g.ldp = p.Np;
   g.tgt = reinterpret_cast<float*>(ws + L.tgt);
-  if (launch_gemm<false, false, kEpiLse>(p.big_s, g, 1, s) != hipSuccess) return MSD_E_HIP;
+  if (launch_gemm<false, false, kEpiLse>(p.big_f, g, 1, s) != hipSuccess) return MSD_E_HIP;
   float* lrow = reinterpret_cast<float*>(ws + L.lrow);
   hipLaunchKernelGGL(xent_lse, dim3((n_rows + 15) / 16), dim3(256), 0, s, reinterpret_cast<const float2*>(g.part),
-                     cdiv(vocab, p.big_s ? 256 : 128), int64_t(p.Np), g.tgt, n_rows, lse, lrow);
+                     cdiv(vocab, p.big_f ? 256 : 128), int64_t(p.Np), g.tgt, n_rows, lse, lrow);
   hipLaunchKernelGGL(xent_mean, dim3(1), dim3(1024), 0, s, lrow, n_rows, loss);
   return hipGetLastError() == hipSuccess ? MSD_OK : MSD_E_HIP;
 }

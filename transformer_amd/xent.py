@@ -13,8 +13,8 @@ the reference's backward casts them (model.py:361).
 What runs (``msd_xent_targets`` / ``msd_xent_forward`` / ``msd_xent_backward``, ``csrc/xent.hip``): the forward streams
 the whole vocabulary through one MFMA GEMM whose epilogue keeps only each row's running
 (max, sum of exponentials), so no logits are stored; the per-row logsumexp is kept for the
-backward.  The backward runs chunk by chunk over the vocabulary (at least ``chunk_size`` columns;
-more while a chunk's block stays within 256 MiB): the softmax block minus the one-hot targets,
+backward.  The backward runs chunk by chunk over the vocabulary (``chunk_size`` bounds the workspace;
+``msd_xent_plan`` gives the columns per chunk): the softmax block minus the one-hot targets,
 scaled by g / N, is formed in bf16 and multiplied into grad_weight (final per chunk) and grad_h
 (f32 partial sums).  Differences from the reference: the forward's logits are f32 sums of exact bf16
 products (the reference's forward runs in the bf16 params dtype), and the backward's softmax
@@ -36,10 +36,15 @@ def _workspace_bytes(n, V, d, chunk):
     return _lib.check(_lib.lib().msd_xent_workspace_bytes(n, V, d, chunk), "msd_xent_workspace_bytes")
 
 
-def _workspace(device, n, V, d, chunk):
+def _workspace(like, n, V, d, chunk):
     """The device workspace of one call, from torch's caching allocator: calls on several streams or
     threads never share one, and the block is used again in stream order once the call has returned."""
-    return torch.empty(_workspace_bytes(n, V, d, chunk), dtype=torch.uint8, device=device)
+    return like.new_empty(_workspace_bytes(n, V, d, chunk), dtype=torch.uint8)
+
+
+def _row_pointers(rows, n):
+    p = rows.data_ptr()
+    return p, p + 4 * n, p + 4 * n + 4
 
 
 def _check_inputs(h, weight, targets):
@@ -65,45 +70,45 @@ class FusedCrossEntropy(torch.autograd.Function):
         N, d = h.shape
         V = weight.shape[0]
         chunk = int(chunk_size)
-        ws = _workspace(h.device, N, V, d, chunk)
+        ws = _workspace(h, N, V, d, chunk)
         loss = torch.empty((), dtype=torch.float32, device=h.device)
-        lse = torch.empty(N, dtype=torch.float32, device=h.device)
-        # int32 targets and the status word behind them
-        tg = torch.empty(N + 1, dtype=torch.int32, device=h.device)
+        # what the backward reads of the forward: int32 targets, the status word, the rows' f32 logsumexp
+        rows = torch.empty(2 * N + 1, dtype=torch.int32, device=h.device)
+        tg, status, lse = _row_pointers(rows, N)
         raw = (targets if targets.dtype in (torch.int32, torch.int64) else targets.to(torch.int64)).contiguous()
         s = torch.cuda.current_stream(h.device)
         stream = ctypes.c_void_p(s.cuda_stream)
-        status = tg.data_ptr() + 4 * N
-        _lib.check(_lib.lib().msd_xent_targets(raw.data_ptr(), raw.element_size(), N, V, tg.data_ptr(), status, stream),
+        _lib.check(_lib.lib().msd_xent_targets(raw.data_ptr(), raw.element_size(), N, V, tg, status, stream),
                    "msd_xent_targets")
         if check_targets:   # the copy back waits for the targets only, while the logits GEMM runs
             host = torch.empty(1, dtype=torch.int32, pin_memory=True)
-            host.copy_(tg[N:], non_blocking=True)
+            host.copy_(rows[N:N + 1], non_blocking=True)
             copied = s.record_event()
-        rc = _lib.lib().msd_xent_forward(h.data_ptr(), weight.data_ptr(), tg.data_ptr(), N, V, d, ws.data_ptr(),
-                                         loss.data_ptr(), lse.data_ptr(), status, stream)
+        rc = _lib.lib().msd_xent_forward(h.data_ptr(), weight.data_ptr(), tg, N, V, d, ws.data_ptr(),
+                                         loss.data_ptr(), lse, status, stream)
         _lib.check(rc, "msd_xent_forward")
         if check_targets:
             copied.synchronize()
             if int(host) & STATUS_BAD_TARGET:
                 raise ValueError(f"a target id outside [0, {V})")
-        ctx.save_for_backward(h, weight, tg, lse)
+        ctx.save_for_backward(h, weight, rows)
         ctx.chunk = chunk
         return loss
 
     @staticmethod
     def backward(ctx, g):
-        h, weight, tg, lse = ctx.saved_tensors
+        h, weight, rows = ctx.saved_tensors
         N, d = h.shape
         V = weight.shape[0]
-        ws = _workspace(h.device, N, V, d, ctx.chunk)
+        ws = _workspace(h, N, V, d, ctx.chunk)
         gl = g.detach().to(torch.float32).reshape(1).contiguous()
         grad_h = torch.empty_like(h)
         grad_w = torch.empty_like(weight)
         s = torch.cuda.current_stream(h.device)
-        rc = _lib.lib().msd_xent_backward(h.data_ptr(), weight.data_ptr(), tg.data_ptr(), lse.data_ptr(),
-                                          gl.data_ptr(), N, V, d, ctx.chunk, ws.data_ptr(), grad_h.data_ptr(),
-                                          grad_w.data_ptr(), tg.data_ptr() + 4 * N, ctypes.c_void_p(s.cuda_stream))
+        tg, status, lse = _row_pointers(rows, N)
+        rc = _lib.lib().msd_xent_backward(h.data_ptr(), weight.data_ptr(), tg, lse, gl.data_ptr(), N, V, d, ctx.chunk,
+                                          ws.data_ptr(), grad_h.data_ptr(), grad_w.data_ptr(), status,
+                                          ctypes.c_void_p(s.cuda_stream))
         _lib.check(rc, "msd_xent_backward")
         ctx.keep = gl
         return grad_h, grad_w, None, None, None
