@@ -7,11 +7,14 @@ f64 arithmetic on the same values is the exact answer.  Tolerances: the loss to 
 block, so each element within 2e-2 relative plus 2e-3 of the largest magnitude, and the whole
 tensor within 5e-3 relative (Frobenius).
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import xent as ox
+from transformer_amd import _lib
 from transformer_amd.xent import fused_cross_entropy, fused_output_and_loss
 
 pytestmark = pytest.mark.gpu
@@ -56,21 +59,39 @@ def _against_oracle(N, V, d, chunk, seed, h_scale=1.0, g=1.0):
           f"grad_h rel {r1:.2e}, grad_weight rel {r2:.2e}")
 
 
+def _plan(N, V, d, chunk):
+    """msd_xent_plan: ids per chunk, chunks, tiles of (forward, logits, grad_weight, grad_h), K splits of
+    grad_h in the first and the last chunk."""
+    out = (ctypes.c_int32 * 8)()
+    _lib.check(_lib.lib().msd_xent_plan(N, V, d, chunk, out), "msd_xent_plan")
+    return tuple(out)
+
+
 def test_ragged_shapes_and_chunks():
-    """Rows and vocabulary not multiples of the 256-tiles, two chunks with a short last one."""
+    """Rows and vocabulary not multiples of the tiles; a single row."""
     _against_oracle(300, 1000, 256, 384, seed=1)
     _against_oracle(1, 77, 128, 4096, seed=2, g=0.5)
 
 
-@pytest.mark.parametrize("N,V,d,chunk", [
-    (65, 257, 128, 100),        # 128-tiles: one row, one id past a tile; token padding to 64
-    (129, 4001, 384, 1000),     # 128-tiles, grad_h split over K with a short last split
-    (1023, 16500, 256, 4096),   # 256-tiles for the logits, 128-tiles for the gradients
-    (4352, 30000, 640, 1000),   # 256-tiles for grad_h with a half-empty last column tile
-    (20000, 7000, 128, 256),    # probability block past its cap: two chunks
+@pytest.mark.parametrize("N,V,d,chunk,plan", [
+    # one row, one id past a tile; token padding to 64
+    (65, 257, 128, 100, (512, 1, 128, 128, 128, 128, 1, 1)),
+    # grad_h split over K with a short last split
+    (129, 4001, 384, 1000, (4096, 1, 128, 128, 128, 128, 8, 8)),
+    (1023, 16500, 256, 4096, (16640, 1, 128, 128, 128, 128, 29, 29)),
+    # 256-tiles for the logits and grad_weight, ragged in tokens and vocabulary
+    (1000, 13800, 1024, 4096, (13824, 1, 256, 256, 256, 128, 8, 8)),
+    # two chunks, the last one short and with fewer splits
+    (3158, 7206, 128, 100, (3840, 2, 128, 128, 128, 128, 7, 6)),
+    # three chunks with 256-tiles for the logits and grad_h, one split fewer in the last
+    (10506, 3087, 256, 256, (1280, 3, 128, 256, 128, 256, 2, 1)),
+    # four chunks, 256-tiles for grad_h with a half-empty last column tile
+    (4352, 30000, 640, 1000, (7680, 4, 256, 256, 128, 256, 5, 5)),
+    (20000, 7000, 128, 256, (1024, 7, 256, 128, 128, 128, 2, 2)),
 ])
-def test_tile_sizes_splits_and_chunks(N, V, d, chunk):
-    """Each tile size of each product, at ragged edges (tolerances as above)."""
+def test_tile_sizes_splits_and_chunks(N, V, d, chunk, plan):
+    """Each tile size of each product, at ragged edges, over one and several chunks (tolerances as above)."""
+    assert _plan(N, V, d, chunk) == plan
     _against_oracle(N, V, d, chunk, seed=8)
 
 
@@ -87,10 +108,10 @@ def test_306m_output_layer_4096_rows():
 def test_chunk_size_changes_only_the_grad_h_summation():
     """grad_weight and the loss are bitwise independent of the chunk size (every element is formed
     the same way); grad_h sums the chunks in f32 and agrees to rounding."""
-    h, w, t = _inputs(700, 5000, 256, seed=5)
-    a = _run(h, w, t, 256)
-    b = _run(h, w, t, 4096)
-    c = _run(h, w, t, 100000)
+    N, V, d, chunks = 8100, 8003, 128, (256, 1000, 100000)
+    assert [_plan(N, V, d, c)[1] for c in chunks] == [3, 2, 1]
+    h, w, t = _inputs(N, V, d, seed=5)
+    a, b, c = (_run(h, w, t, c) for c in chunks)
     assert a[0] == b[0] == c[0]
     assert np.array_equal(a[2], b[2]) and np.array_equal(b[2], c[2])
     np.testing.assert_allclose(a[1], c[1], rtol=1e-2, atol=1e-3 * np.abs(c[1]).max())

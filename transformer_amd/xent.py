@@ -101,7 +101,7 @@ class FusedCrossEntropy(torch.autograd.Function):
         N, d = h.shape
         V = weight.shape[0]
         ws = _workspace(h, N, V, d, ctx.chunk)
-        gl = g.detach().to(torch.float32).reshape(1).contiguous()
+        gl = g if g.dtype == torch.float32 else g.detach().to(torch.float32)   # a scalar
         grad_h = torch.empty_like(h)
         grad_w = torch.empty_like(weight)
         s = torch.cuda.current_stream(h.device)
