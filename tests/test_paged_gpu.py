@@ -210,6 +210,48 @@ def test_bad_positions_and_pages_are_reported():
     assert out[1] & 4
 
 
+@pytest.mark.parametrize("B", [9, 65, 600])
+def test_multi_kernel_step_reports_bad_rows_and_recovers(B):
+    """Past 8 sequences: every row's flags are gathered from one word per row and kind (600 rows: more
+    than a workgroup's threads), a bad row leaves the others alone, and the next step starts clean."""
+    w = prepare_decode_weights_nlayer(make_params(TINY, seed=0), TINY)
+    pool = PagePool(TINY, B + 1)   # page 0, which a bad entry is replaced by, belongs to no sequence
+    cached = torch.randn(pool.data.shape, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+    bd = PagedBatchDecoder(w, TINY, pool, B)
+    rng = np.random.default_rng(4)
+    bd.tables[:, 0] = torch.from_numpy(1 + rng.permutation(B).astype(np.int32)).cuda()
+    toks = torch.from_numpy(rng.integers(0, TINY["vocab_size"], B).astype(np.int32)).cuda()
+    pos = torch.from_numpy(rng.integers(0, PAGE, B).astype(np.int32)).cuda()
+
+    def step(want, bad=None):
+        pool.data.copy_(cached)   # (a row whose position is replaced by 0 stores its K/V there)
+        out = bd.launch(toks, pos).cpu().numpy()
+        assert np.array_equal(out[1::2], np.full(B, want)), (want, out[1::2][:8])
+        lg = bd.logits.clone()
+        if bad is not None:
+            keep = torch.arange(B, device="cuda") != bad
+            assert torch.equal(lg[keep], good[keep])
+        return lg
+
+    def spoil(t, at, value, want, row):
+        old = t[at].clone()
+        t[at] = value
+        step(want, row)
+        t[at] = old
+
+    good = step(0)
+    for row in (0, B // 2, B - 1):
+        for value in (-1, TINY["context_len"], 10 ** 6):
+            spoil(pos, row, value, 4, row)
+        for value in (-1, TINY["vocab_size"]):
+            spoil(toks, row, value, 2, row)
+        for value in (-1, B + 1):
+            spoil(bd.tables, (row, 0), value, 4, row)
+        spoil(bd.tables, (row, 1), -1, 0, None)   # a page past the row's position is not used
+    toks[0], pos[B - 1] = -1, -1
+    step(6)
+
+
 def test_persistent_step_matches_multi_kernel_step():
     """Up to 8 sequences step in one persistent launch; 9 take the multi-kernel pass.  The same
     8 sequences through both agree (different summation orders: 1e-4), with the same tokens."""
