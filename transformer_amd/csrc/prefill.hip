@@ -1140,10 +1140,12 @@ __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const flo
   }
 }
 
-// Four heads of a K/V head per workgroup when that still leaves a workgroup per CU: the K/V rows are
-// then read once for the four (306M, 64 rows: 1004 -> 943 us per step); with fewer workgroups the idle
-// CUs cost more than the shared reads save (24 rows: 803 us with one head, 806 with two, 859 with
-// four).
+// Four heads of a K/V head per workgroup read its K/V rows once, but their workgroups take four times as
+// long, so the last pass over the CUs has to be nearly full (7/8): measured per step at 12..100 / 48..384
+// positions, four heads against one: 306M 64 rows (256 workgroups) 0.950 / 0.937, 56 (224) 0.966 / 0.973,
+// 128 (512) 0.941 / 0.956, 40 (160) 0.983 / 1.013, 96 (384) 1.013 / 1.027, 72 (288) 1.044 / 1.051;
+// 512 wide with 8 heads, 128 rows (256) 0.980 / 0.963, 96 (192) 1.003 / 1.019, 160 (320) 1.042 / 1.069.
+// (Two heads, 24 rows of the 306M: 806 us against 803 with one and 859 with four.)
 static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const float* qkv, const Rows& rows,
                                     const uint16_t* kc, const uint16_t* vc, uint16_t* att, int64_t plane,
                                     int natural) {
@@ -1151,7 +1153,8 @@ static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const f
   auto go = [&](auto k, int gh) {
     hipLaunchKernelGGL(k, dim3(M, H / gh), dim3(64 * kAttnWaves), 0, s, qkv, rows, H, KV, kc, vc, att, plane, 0, natural);
   };
-  if (G % 4 == 0 && M * H / 4 >= 256) go(mx_attention_decode<4>, 4);
+  const int last = (M * H / 4 + 255) % 256 + 1;   // workgroups of the last pass
+  if (G % 4 == 0 && last >= 224) go(mx_attention_decode<4>, 4);
   else go(mx_attention_decode<1>, 1);
 }
 
