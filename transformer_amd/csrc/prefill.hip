@@ -1663,15 +1663,18 @@ static int64_t first_norm_scales(const msd_config* c) {
 }
 
 // Weights that do not fit the 256 MB last-level cache (tile copies past kCacheBytes) are split: the first
-// layers, up to kKeepBytes, are read with the default policy and stay there from one pass to the
-// next, the others non-temporal, so they stream past. Measured at 306M (541 MB; none / 90 / 130 / 160
-// MiB kept): verification of 5 tokens 646 / 604 / 595 / 593 us, prefill of 16 686 / 643 / 632 / 629, of
-// 64 722 / 685 / 676 / 675, of 128 849 / 834 / 823 / 817. Past 128 rows it loses (200 rows 1095 / 1170 /
-// 1149 / 1141: a weight tile then serves many row tiles' workgroups, and its lines leave the L2 before
-// the last has read them), and a batched step's own K/V rows (127 MB for 24 sequences) need the
-// cache (735 / 729 / 737 / 739): both keep the default policy throughout.
+// layers, up to kKeepBytes, are read with the default policy and stay there until the next pass, the
+// others non-temporal, so they stream past.  That gains between passes that follow each other (chunks
+// of a prompt, drafts and their verification) and nothing after a decode step, which streams its own
+// copy of the weights.  Measured at 306M (541 MB; default policy / split, passes in a row and each after
+// a decode step): verification of 5 tokens 664 / 603 and 670 / 668 us, prefill of 16 691 / 641 and
+// 706 / 705, of 64 739 / 695 and 754 / 758, but of 128 870 / 841 and 879 / 908: at more rows a weight tile
+// serves more row tiles' workgroups, and its lines leave the L2 before the last has read them (200 rows
+// in a row 1124 / 1182).  So kStreamRows is the largest that loses nothing in either order.
+// A batched step keeps the default policy: its own K/V rows want the cache, and the host does not know the
+// positions (9 sequences of up to 40 positions 709 / 653 us, but 24 of up to 384 751 / 756, 48 926 / 952).
 constexpr int64_t kKeepBytes = int64_t(150) << 20, kCacheBytes = int64_t(224) << 20;
-constexpr int kStreamRows = 128;
+constexpr int kStreamRows = 64;
 
 // The layer stack over M rows whose residual stream is already in h; leaves the last
 // projection's partials pending (returned split count).
