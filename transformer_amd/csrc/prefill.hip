@@ -235,9 +235,9 @@ __device__ __forceinline__ f32x4 mfma3(uint4 ah, uint4 al, uint4 bh, uint4 bl, f
 }
 
 
-// Four waves as WM x (4 / WM); a wave covers RB 16-row blocks and (WM) 16-column blocks.  TA / TW:
-// the activations / weights in tile order (one 1 KB piece per operand load).
-template <int RB, int WM, bool TA, bool TW>
+// Four waves as WM x (4 / WM); a wave covers RB 16-row blocks and (WM) 16-column blocks.  TA:
+// the activations in tile order (one 1 KB piece per operand load); the weights are in row order.
+template <int RB, int WM, bool TA>
 __global__ __launch_bounds__(256) void mx_gemm(GemmArgs g) {
   constexpr int WN = 4 / WM, CB = 4 / WN, BM = 16 * RB * WM;
   constexpr int U = RB * CB <= 2 ? 8 : 4;   // K steps with loads in flight
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void mx_gemm(GemmArgs g) {
   const int c0 = (nchunks * int(blockIdx.z)) / g.splits, c1 = (nchunks * (int(blockIdx.z) + 1)) / g.splits;
   const int kq = 8 * (lane >> 4);   // this lane's 8-element K run within a 32 chunk
   const int r16 = lane & 15;
-  // operand pointers of chunk 0; chunk c is kstep(c) elements further
+  // operand pointers of chunk 0
   const uint16_t* arow[RB];   // hi parts (the lo parts a_plane elements further)
   bool aval[RB];
 #pragma unroll
@@ -263,9 +263,7 @@ __global__ __launch_bounds__(256) void mx_gemm(GemmArgs g) {
   const uint16_t* wrow[CB];
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb)
-    wrow[cb] = TW ? g.W + (int64_t((n0 + 16 * cb) >> 4) * nchunks * 64 + lane) * 8
-                  : g.W + int64_t(n0 + 16 * cb + r16) * g.K + kq;
-  auto kstep = [](int c, bool tiled) { return tiled ? int64_t(c) * 512 : int64_t(c) * kBK; };
+    wrow[cb] = g.W + int64_t(n0 + 16 * cb + r16) * g.K + kq;
   f32x4 acc[RB][CB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
@@ -288,7 +286,7 @@ __global__ __launch_bounds__(256) void mx_gemm(GemmArgs g) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int ch = min(c + u, c1 - 1);
-      const int64_t ka = kstep(ch, TA), kw = kstep(ch, TW);
+      const int64_t ka = int64_t(ch) * (TA ? 512 : kBK), kw = int64_t(ch) * kBK;
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         const uint4 v = *reinterpret_cast<const uint4*>(arow[rb] + ka);
@@ -390,10 +388,10 @@ __device__ __forceinline__ uint4 load_w(const uint16_t* p) {
 // flight; the waves' tiles are added through LDS in wave order, row tile by row tile, so the result
 // is deterministic.  Tiles are dealt XCD-aware: each XCD (workgroup b runs on XCD b mod 8) takes a
 // contiguous range of the tiles, row tiles innermost, so a column group's weights reach its L2 once.
-// AM: the A operand as bf16 hi/lo rows (0) or tiles (1) as for mx_gemm, or (2) RMSNorm folded in
-// (model.py:94-98): A = the hi/lo tiles of scale * h that the previous projection's
+// AM: the A operand as bf16 hi/lo tiles (1), or (2) RMSNorm folded in (model.py:94-98): A = the hi/lo tiles of scale * h that the previous projection's
 // epilogue wrote (kEpiResid), and every output divided by sqrt(mean(h^2) + 1e-5), the sum of
-// h^2 of each row added up from that epilogue's per-column-group partials.  TW as for mx_gemm.
+// h^2 of each row added up from that epilogue's per-column-group partials.  TW: the weights in tile
+// order (else in row order).
 // EPI: store the outputs, add them to the residual out (tile order; with an act plane also the
 // hi/lo tiles of scale * h and the row's partial sum of h^2 for the next RMSNorm), or finish them
 // in place of mx_swiglu_fin / mx_qkv_fin (the same arithmetic).
@@ -402,7 +400,7 @@ __device__ __forceinline__ uint4 load_w(const uint16_t* p) {
 // NT: the weights are read non-temporal (layers past kKeepBytes).
 template <int RT, int CT, int P, int NW, int AM, bool TW, int EPI, bool NT = false>
 __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
-  static_assert(RT == 1 || (AM >= 1 && TW), "several row tiles per workgroup: tile-order operands");
+  static_assert(RT == 1 || TW, "several row tiles per workgroup: tile-order weights");
   // the waves' partial tiles of one row tile, a lane's four outputs as one 16-byte piece (written and
   // read across lanes contiguously); two buffers, so one barrier per row tile suffices
   __shared__ f32x4 red[RT > 1 ? 2 : 1][NW][CT][64];
@@ -425,12 +423,11 @@ __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int tile = min(RT * t + rt, T - 1);
-    ar[rt] = AM >= 1 ? g.A + (int64_t(tile) * S * 64 + min(r16, g.M - 1 - 16 * tile) + 16 * (lane >> 4)) * 8
-                     : g.A + int64_t(min(m0 + r16, g.M - 1)) * g.lda + kq;
+    ar[rt] = g.A + (int64_t(tile) * S * 64 + min(r16, g.M - 1 - 16 * tile) + 16 * (lane >> 4)) * 8;
   }
   const uint16_t* wr = TW ? g.W + (int64_t(n0 >> 4) * S * 64 + lane) * 8 : g.W + int64_t(n0 + r16) * g.K + kq;
   // element offsets of step ks and of column tile ct
-  const int64_t astep = AM >= 1 ? 512 : kBK, wstep = TW ? 512 : kBK;
+  const int64_t astep = 512, wstep = TW ? 512 : kBK;
   const int64_t wtile = TW ? int64_t(S) * 512 : int64_t(16) * g.K;
   const int ns = (S - wv + NW - 1) / NW;   // K steps of this wave (possibly none)
   f32x4 acc[RT][CT];
@@ -743,7 +740,7 @@ __global__ __launch_bounds__(256) void mx_qkv_fin(const float* part, int splits,
 // Row blockIdx.x: act_f = silu(gate_f) * up_f over the summed partials (gate/up are the packed
 // rows 2f, 2f+1; model.py:159), as hi/lo bf16 parts at the down projection's input position of f.
 __global__ __launch_bounds__(256) void mx_swiglu_fin(const float* part, int splits, int M, int F, uint16_t* act,
-                                                     int64_t plane, int ldx) {
+                                                     int64_t plane) {
   const int m = blockIdx.x, f = 2 * (blockIdx.y * 256 + threadIdx.x);   // outputs f and f + 1 (F is even)
   if (f >= F) return;
   float4 pv[kMaxSplitK];
@@ -759,8 +756,8 @@ __global__ __launch_bounds__(256) void mx_swiglu_fin(const float* part, int spli
       g1 += pv[z].z;
       u1 += pv[z].w;
     }
-  put_split(act + act_index(m, perm_pos(f, F), F, ldx), plane, swiglu(g0, u0));
-  put_split(act + act_index(m, perm_pos(f + 1, F), F, ldx), plane, swiglu(g1, u1));
+  put_split(act + act_index(m, perm_pos(f, F), F, 0), plane, swiglu(g0, u0));
+  put_split(act + act_index(m, perm_pos(f + 1, F), F, 0), plane, swiglu(g1, u1));
 }
 
 // Reductions over the 16 lanes of a DPP row, every lane receiving the result (rotations by 1, 2,
@@ -977,8 +974,7 @@ __device__ __forceinline__ float sum8_lanes(float v) {   // over each 8 consecut
 template <int GH>
 __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const float* qkv, Rows rows, int H, int KV,
                                                                        const uint16_t* kc, const uint16_t* vc,
-                                                                       uint16_t* att, int64_t plane, int ldx,
-                                                                       int natural) {
+                                                                       uint16_t* att, int64_t plane, int natural) {
   // per wave and row of 16 lanes: the output's partial sums and the softmax denominator's
   __shared__ float so[kAttnWaves][4][GH][kDh];
   __shared__ float sl[kAttnWaves][4][GH];
@@ -1130,12 +1126,12 @@ __global__ __launch_bounds__(64 * kAttnWaves) void mx_attention_decode(const flo
     if (natural) {
       uint32_t hi, lo;
       split2(num0, num1, hi, lo);
-      const int64_t at = act_index(m, el, d, ldx);
+      const int64_t at = act_index(m, el, d, 0);
       *reinterpret_cast<uint32_t*>(att + at) = hi;
       *reinterpret_cast<uint32_t*>(att + plane + at) = lo;
     } else {
-      put_split(att + act_index(m, perm_pos(el, d), d, ldx), plane, num0);
-      put_split(att + act_index(m, perm_pos(el + 1, d), d, ldx), plane, num1);
+      put_split(att + act_index(m, perm_pos(el, d), d, 0), plane, num0);
+      put_split(att + act_index(m, perm_pos(el + 1, d), d, 0), plane, num1);
     }
   }
 }
@@ -1151,7 +1147,7 @@ static void launch_attention_decode(int M, int H, int KV, hipStream_t s, const f
                                     int natural) {
   const int G = H / KV;
   auto go = [&](auto k, int gh) {
-    hipLaunchKernelGGL(k, dim3(M, H / gh), dim3(64 * kAttnWaves), 0, s, qkv, rows, H, KV, kc, vc, att, plane, 0, natural);
+    hipLaunchKernelGGL(k, dim3(M, H / gh), dim3(64 * kAttnWaves), 0, s, qkv, rows, H, KV, kc, vc, att, plane, natural);
   };
   const int last = (M * H / 4 + 255) % 256 + 1;   // workgroups of the last pass
   if (G % 4 == 0 && last >= 224) go(mx_attention_decode<4>, 4);
@@ -1438,8 +1434,8 @@ static int rows_ct(int M, int N, int K) {
 struct RowsTile {
   int rt, ct, nw;   // row tiles, column tiles, waves
 };
-constexpr RowsTile kRowsTiles[] = {{1, 1, 8}, {1, 1, 4}, {1, 2, 4}, {1, 3, 4}, {1, 4, 4}, {1, 6, 4}, {2, 2, 4},
-                                   {2, 3, 4}, {2, 4, 4}, {2, 6, 4}, {4, 3, 4}, {4, 4, 4}, {4, 6, 4}, {4, 11, 4}};
+constexpr RowsTile kRowsTiles[] = {{1, 1, 8}, {1, 1, 4}, {1, 2, 4}, {1, 3, 4}, {1, 4, 4}, {1, 6, 4},
+                                   {2, 3, 4}, {2, 4, 4}, {2, 6, 4}, {4, 4, 4}, {4, 6, 4}, {4, 11, 4}};
 
 // The tile of a projection, from a model of its time (us) fitted to cold-weight runs of the 306M
 // projections at 5..511 rows (within ~10 % of each; e.g. 511-row gate/up: 4 x 11 19.0 us, 2 x 6
@@ -1571,20 +1567,25 @@ static void launch_rows_tiles(const RowsTile& t, int grid, hipStream_t s, const 
   constexpr RowsTile k = kRowsTiles[I];
   if (t.rt == k.rt && t.ct == k.ct && t.nw == k.nw) {
     constexpr int P = k.rt * k.ct == 1 && k.nw == 4 && EPI == kEpiResid ? 8 : k.rt == 1 && k.ct <= 4 ? 4 : (k.rt * k.ct <= 6 ? 3 : 2);
-    if (nt)
-      hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI, true>), dim3(grid), dim3(64 * k.nw), 0, s, g);
-    else
-      hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI>), dim3(grid), dim3(64 * k.nw), 0, s, g);
+    // (the tiles that passes of up to kStreamRows rows take have a non-temporal form)
+    constexpr bool kNt = EPI == kEpiSwiglu ? k.rt <= 2 : k.rt == 1 && k.ct <= (EPI == kEpiQkv ? 3 : 1);
+    if constexpr (kNt) {
+      if (nt) {
+        hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI, true>), dim3(grid), dim3(64 * k.nw), 0, s, g);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((mx_gemm_rows<k.rt, k.ct, P, k.nw, AM, true, EPI>), dim3(grid), dim3(64 * k.nw), 0, s, g);
   } else if constexpr (I + 1 < int(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))) {
     launch_rows_tiles<AM, EPI, I + 1>(t, grid, s, g, nt);
   }
 }
 
-template <bool TA, bool TW>
+template <bool TA>
 static void launch_splitk(int bm, dim3 grid, hipStream_t s, const GemmArgs& g) {
-  if (bm == 16) hipLaunchKernelGGL((mx_gemm<1, 1, TA, TW>), grid, dim3(256), 0, s, g);
-  else if (bm == 64) hipLaunchKernelGGL((mx_gemm<2, 2, TA, TW>), grid, dim3(256), 0, s, g);
-  else hipLaunchKernelGGL((mx_gemm<4, 2, TA, TW>), grid, dim3(256), 0, s, g);
+  if (bm == 16) hipLaunchKernelGGL((mx_gemm<1, 1, TA>), grid, dim3(256), 0, s, g);
+  else if (bm == 64) hipLaunchKernelGGL((mx_gemm<2, 2, TA>), grid, dim3(256), 0, s, g);
+  else hipLaunchKernelGGL((mx_gemm<4, 2, TA>), grid, dim3(256), 0, s, g);
 }
 
 // C = A W^T split over K: partials [splits][M][N] (pass ldo = N), or with splits == 1 rows
@@ -1620,8 +1621,8 @@ static hipError_t gemm(const uint16_t* A, int64_t a_plane, int lda, const uint16
   }
   const int bm = bm_for(M);
   const dim3 grid(N / kBN, (M + bm - 1) / bm, splits);
-  if (am == 1) launch_splitk<true, false>(bm, grid, s, g);
-  else launch_splitk<false, false>(bm, grid, s, g);
+  if (am == 1) launch_splitk<true>(bm, grid, s, g);
+  else launch_splitk<false>(bm, grid, s, g);
   return hipGetLastError();
 }
 
@@ -1771,7 +1772,7 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
     if ((err = gemm(att, pd, 0, Wl + off_o, false, M, d, d, part, d, so, s)) != hipSuccess) break;
     hipLaunchKernelGGL(mx_norm, dim3(M), dim3(kNormThreads), 0, s, h, part, so, M, d, Wl + off_ln2, xn, pd, 0, 0, 0);
     if ((err = gemm(xn, pd, 0, Wl + off_gu, false, M, 2 * ff, d, part, 2 * ff, sg, s)) != hipSuccess) break;
-    hipLaunchKernelGGL(mx_swiglu_fin, dim3(M, (ff / 2 + 255) / 256), dim3(256), 0, s, part, sg, M, ff, act, pf, 0);
+    hipLaunchKernelGGL(mx_swiglu_fin, dim3(M, (ff / 2 + 255) / 256), dim3(256), 0, s, part, sg, M, ff, act, pf);
     if ((err = gemm(act, pf, 0, Wl + off_dn, false, M, d, ff, part, d, sd, s)) != hipSuccess) break;
     pending = sd;
   }
