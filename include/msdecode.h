@@ -253,10 +253,10 @@ int32_t msd_prefill(const msd_config* cfg, const void* token_emb, const void* ou
 
 /* Launch mode of the multi-row passes (msd_prefill, msd_prefill_paged, msd_verify and the
  * multi-kernel pass of msd_batch_decode_step).  With graphs on (off by default; the environment
- * variable MSD_LAUNCH_GRAPHS=1 starts with them on) the ~130 dependent launches of a pass are
+ * variable MSD_LAUNCH_GRAPHS=1 starts with them on) the ~125 dependent launches of a pass are
  * captured once per argument set (shape, device pointers, sizes) into a HIP graph that is kept
  * (at most 16 per process, the least recently used dropped) and replayed on the caller's stream.
- * That cuts the host's enqueue time per pass from ~0.35 to ~0.07 ms (306M) but runs ~1 % slower
+ * That cuts the host's enqueue time per pass from ~0.32 to ~0.09 ms (306M) but runs ~1 % slower
  * on the device, so it is for callers whose host thread is the bottleneck.  Buffer contents are
  * read when the kernels run, so a pass over new tokens in the same buffers replays the same
  * graph.  A stream the caller is capturing gets the launches directly.  Results are bitwise the

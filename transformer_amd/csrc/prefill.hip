@@ -20,7 +20,9 @@
 // A row's position p lives at page table[p / 16] * 16 + p % 16; without a table the page is
 // p / 16 (the contiguous cache of one sequence is the pool with the identity table).
 //
-// Kernels per layer, on the caller's stream:
+// With the tile copy of the weights (msd_pack_tiles) a layer is five kernels on the caller's stream: mx_gemm_rows
+// for QKV, O, gate/up and down, with the norms, RoPE, SwiGLU and the residual in its epilogues, and the
+// attention (run_layers).  Without it:
 //   mx_norm        residual += split-K partials of the previous projection (in split order),
 //                  then RMSNorm -> bf16 activations in the weights' permuted input order
 //   mx_gemm        q/k/v projection, split-K partials
@@ -33,9 +35,10 @@
 //   mx_gemm        gate/up projection, split-K partials
 //   mx_swiglu_fin  silu(gate) * up -> bf16 in the down projection's input order
 //   mx_gemm        down projection, split-K partials
-// then mx_norm with the final scale, mx_gemm against the tied embedding, mx_argmax per row.
+// Either way then mx_norm with the final scale, the tied logits (mx_gemm for one row, mx_logits for more) and
+// mx_argmax per row.
 //
-// GEMM: C[M x N] = A[M x K] * W[N x K]^T with A (activations) and W (packed weight rows)
+// mx_gemm: C[M x N] = A[M x K] * W[N x K]^T with A (activations) and W (packed weight rows)
 // both K-contiguous.  A workgroup of four waves covers 64 columns and BM rows; each wave
 // holds RB x CB 16 x 16 MFMA tiles, every operand fragment one 16-byte run along K loaded
 // straight from memory (W streamed once per row tile, A from L2).  K is split across grid.z
@@ -396,7 +399,7 @@ __device__ __forceinline__ uint4 load_w(const uint16_t* p) {
 // hi/lo tiles of scale * h and the row's partial sum of h^2 for the next RMSNorm), or finish them
 // in place of mx_swiglu_fin / mx_qkv_fin (the same arithmetic).
 // Measured at 306M in the pass (one 16-row tile per workgroup and scalar epilogues before): gate/up of
-// 511 rows 31.8 -> 18.8 us, of 128 11.8 -> 10.2, of 5 7.2 -> 5.3; what bounds it is in rows_tile.
+// 511 rows 31.8 -> 20.6 us, of 128 11.8 -> 10.7, of 5 7.2 -> 5.5; what bounds it is in rows_tile.
 // NT: the weights are read non-temporal (layers past kKeepBytes).
 template <int RT, int CT, int P, int NW, int AM, bool TW, int EPI, bool NT = false>
 __global__ __launch_bounds__(64 * NW) void mx_gemm_rows(GemmArgs g) {
@@ -780,9 +783,9 @@ __device__ __forceinline__ float row16_sum(float v) {
 }
 
 // Prefill: causal GQA attention of query block blockIdx.y (16 rows) for head blockIdx.x on the
-// matrix cores.  The key range 0..q0+15 is cut into 32-key chunks, wave w taking chunks w, w + 4,
+// matrix cores.  The key range 0..q0+15 is cut into 32-key chunks, wave w taking chunks w, w + NW,
 // ...: S = Q K^T (16 x 32) and O += P V (16 x 64) run on v_mfma_f32_16x16x32_bf16 with every f32
-// operand as hi/lo bf16 parts (mfma3), the softmax is online per query row in f32, and the four
+// operand as hi/lo bf16 parts (mfma3), the softmax is online per query row in f32, and the NW
 // waves' (max, sum, O) are merged by log-sum-exp at the end.  Scale 1/sqrt(64) (model.py:98).
 // MFMA operand lanes: A[i][8 (l / 16) ..] = row i = l % 16; B[8 (l / 16) ..][n] with n = l % 16;
 // D: rows 4 (l / 16) + r of column l % 16.
@@ -790,8 +793,9 @@ __device__ __forceinline__ float row16_sum(float v) {
 // natural at their element index (the tile copy's O columns are in natural order).  K and V come as
 // operand planes from the QKV epilogue, so a chunk is 16 loads of 1 KB and no conversion (reading f32
 // rows took 40 loads of 64-byte segments and eight splits per chunk in every head and query block:
-// 511 rows 15.9 us, now 9.5; 128 rows 6.6, now 4.4).  Eight waves past 128 rows (511 rows of f32: 17.1
-// us with four, 15.9 with eight), four where no wave of eight would have a second chunk.
+// 511 rows 17.2 us, now 8.8; 200 rows 8.5, now 5.7; 128 rows 6.6, now 4.9).  Eight waves past 128 rows
+// (mean of 24 layers, eight / four: 200 rows 5.6 / 5.9 us, 511 9.0 / 8.9), four where no wave of eight
+// would have a second chunk.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv, const uint16_t* kvp, int MP, int M, int H,
                                                                 int KV, uint16_t* att, int64_t plane, int natural) {
@@ -805,7 +809,7 @@ __global__ __launch_bounds__(64 * NW) void mx_attention_prefill(const float* qkv
   const int nqkv = (H + 2 * KV) * kDh, d = H * kDh;
   // the first half of the grid takes the later query blocks, latest first, the second half the earlier
   // ones, earliest first: two workgroups half a grid apart, which tend to share a CU, then have
-  // about the same number of chunks together on every CU (511 rows: 9.5 -> 8.0 us)
+  // about the same number of chunks together on every CU (511 rows: 10.2 -> 8.8 us, 200: 5.8 -> 5.7)
   const int half = gridDim.y / 2;
   const int q0 = 16 * (int(blockIdx.y) < half ? int(gridDim.y) - 1 - int(blockIdx.y) : int(blockIdx.y) - half);
   const int nk = min(q0 + 16, M), nch = (nk + 31) / 32;
@@ -960,12 +964,13 @@ static void launch_attention_prefill(int M, int H, int KV, hipStream_t s, const 
 // before the current one's arithmetic.  Lane l reads dims 8 (l % 8) .. + 8 of position 8 i + l / 8, i = 0..3,
 // of K and of V: whole rows, 1 KB per instruction (a lane per position for K and per dim for V took
 // 72 instructions per 64 positions and 64 cache lines per K instruction: 13.9 us for the 24 rows, now
-// 8.2; 5 rows at position 211: 7.4, now 5.4).  The
+// 8.4; 5 rows at position 211: 7.4, now 5.4).  The
 // 8 lanes of a position add their partial scores with DPP, so every lane ends up with the weights of
 // exactly the V rows it holds; only (max, sum, output) partials go through LDS at the end.
 constexpr int kAttnWaves = 8;
-// Positions mx_attention_decode covers.
-constexpr int kAttnMaxCtx = 2048;
+// The longest context of verification and batched decode: that of the decode step whose rows they stand for
+// (msdecode.hip).  The kernel itself streams blocks and has no bound of its own.
+constexpr int kDecodeMaxCtx = 2048;
 __device__ __forceinline__ float sum8_lanes(float v) {   // over each 8 consecutive lanes, as sum16_lanes
   v += dpp<0xB1, 0xf>(v, 0.f);
   v += dpp<0x4E, 0xf>(v, 0.f);
@@ -1439,8 +1444,11 @@ constexpr RowsTile kRowsTiles[] = {{1, 1, 8}, {1, 1, 4}, {1, 2, 4}, {1, 3, 4}, {
 
 // The tile of a projection, from a model of its time (us) fitted to cold-weight runs of the 306M
 // projections at 5..511 rows (within ~10 % of each; e.g. 511-row gate/up: 4 x 11 19.0 us, 2 x 6
-// 20.5, 4 x 6 25.2, 1 x 8 -- the old choice -- 27.4; 128-row gate/up 2 x 6 8.9, 1 x 3 11.2; 24-row
-// 1 x 3 5.7, 1 x 2 6.9): launch, first loads and drain 2.6; every K step moves 2 RT + CT operand
+// 20.5, 4 x 6 25.2, 1 x 8 27.4; 128-row gate/up 2 x 6 8.9, 1 x 3 11.2; 24-row 1 x 3 5.7, 1 x 2 6.9).
+// The widest entry is 11 column tiles because the 306M's gate/up has 352: from 449 rows (8 row groups of
+// 4) on, 11 make one workgroup per CU, 12 leave 16 CUs idle (passes of 383 and 511 rows 1568 / 1569 us
+// with 11, 1576 / 1584 with 12; the other models' passes within 1 % either way) and 10 take a second
+// pass over the CUs.  The model: launch, first loads and drain 2.6; every K step moves 2 RT + CT operand
 // fragments into the CU (13 ns each); the epilogue takes 0.19 per tile; workgroups past one per
 // CU cost a share of both where two fit a CU's registers (up to 12 tiles), whole passes where not.
 // max_groups: an upper limit on column groups (0: none).
@@ -1781,9 +1789,9 @@ static int run_layers(const msd_config* cfg, const Weights& wt, const Rows& rows
 }
 
 // ---- Replaying a pass's launches from a graph (opt-in) ----
-// A pass is ~130 dependent launches; enqueueing them costs the host ~0.35 ms per pass (306M),
-// replaying them from a graph ~0.07 ms.  The device runs the replay ~1 % slower (128-token
-// prefill 1.037-1.047 vs 1.022-1.032 ms; 16 tokens 0.797 vs 0.787 ms), so graphs are for callers
+// A pass is ~125 dependent launches; enqueueing them costs the host ~0.32 ms per pass (306M),
+// replaying them from a graph ~0.09 ms.  The device runs the replay ~1 % slower (128-token
+// prefill 0.872 vs 0.863 ms; 64 tokens 0.703 vs 0.694, 16 0.651 vs 0.642), so graphs are for callers
 // whose host thread is the bottleneck and are off unless asked for (msd_set_launch_graphs, or
 // MSD_LAUNCH_GRAPHS=1 in the environment).  The key holds every value a launch bakes in (shape, device pointers, sizes); buffer
 // contents are read when the kernels run, so a replay with new tokens or weights in the same
@@ -1907,7 +1915,7 @@ static int32_t prefill_impl(const msd_config* cfg, const Weights& wt, const int3
   if (!mx_config_ok(cfg)) return MSD_E_CONFIG;
   const int M = n_tokens;
   if (M <= 0 || start < 0 || start + M > cfg->context_len) return MSD_E_ARG;
-  if (start > 0 && cfg->context_len > kAttnMaxCtx) return MSD_E_CONFIG;   // decode attention
+  if (start > 0 && cfg->context_len > kDecodeMaxCtx) return MSD_E_CONFIG;
   if (argmax_all && !logits_all) return MSD_E_ARG;
   if (!wt.emb || !wt.outp || !wt.w || !wt.lnf || !wt.rope || !tokens || !kv || !workspace || !logits_last ||
       !next_token)
@@ -2058,7 +2066,7 @@ extern "C" int32_t msd_batch_decode_step(const msd_config* cfg, const void* toke
       !aligned16(workspace) || !aligned16(tiles))
     return MSD_E_ARG;
   if (max_pages <= 0 || max_pages > (cfg->context_len + kPage - 1) / kPage || pool_pages <= 0) return MSD_E_ARG;
-  if (cfg->context_len > kAttnMaxCtx) return MSD_E_CONFIG;   // decode attention
+  if (cfg->context_len > kDecodeMaxCtx) return MSD_E_CONFIG;
   hipStream_t s = static_cast<hipStream_t>(stream);
   {   // up to 8 sequences: one persistent launch when the shape and the device allow it
     const mbd::StepArgs sa{cfg, static_cast<const uint16_t*>(token_emb), static_cast<const uint16_t*>(output_proj),
@@ -2110,7 +2118,7 @@ extern "C" int32_t msd_config_support(const msd_config* cfg, int32_t n_workgroup
   if (msdc::decode_supported(cfg, G)) paths |= MSD_PATH_DECODE;
   if (mx_config_ok(cfg)) {
     paths |= MSD_PATH_PREFILL;
-    if (cfg->context_len <= kAttnMaxCtx) paths |= MSD_PATH_VERIFY | MSD_PATH_BATCHED;
+    if (cfg->context_len <= kDecodeMaxCtx) paths |= MSD_PATH_VERIFY | MSD_PATH_BATCHED;
     if ((paths & MSD_PATH_BATCHED) && mbd::region_bytes(cfg) > 0) paths |= MSD_PATH_BATCHED_STEP;
   }
   if (msdc::sample_supported(cfg->vocab_size)) paths |= MSD_PATH_SAMPLE;

@@ -40,10 +40,10 @@
 // of MFMA).  K advances 32 at a time through a ring of 4 LDS stages filled by direct DMA
 // (global_load_lds, 16 bytes per lane); a wave reads the fragments of stage k + 1 while the matrix
 // cores work on stage k, one barrier per stage.
-// Measured (N 4096, V 32000, d 1024; 268 GFLOP per product): forward 307 us (8 waves of 128 x 64,
-// fragments read stage by stage: 329), probabilities 330 (8 chunks: 450 with P and P^T), grad_W
-// 266 (400 in 128-tiles), grad_h 267 + 12 for the partials' sum (520 in 128-tiles, 8 chunks); the
-// two copies W^T and h^T (26 us) are gone.  Timing-only copies without the operand DMA or without
+// Measured (N 4096, V 32000, d 1024, one chunk; 268 GFLOP per product): forward 306 us (8 waves of 128 x 64,
+// fragments read stage by stage: 329), probabilities 328 (8 chunks: 450 with P and P^T), grad_W
+// 253 (128-tiles 304), grad_h 259 + 12 for the partials' sum (128-tiles 340); W^T and h^T are not
+// copied.  Timing-only copies without the operand DMA or without
 // the fragment reads take 207 us per gradient: what is left is the matrix cores at their
 // sustained rate (a large library product: 1.21 PFLOP/s = 221 us) and the epilogues, which one
 // workgroup per CU does not overlap.
@@ -700,8 +700,11 @@ int rup(int x, int m) { return (x + m - 1) / m * m; }
 // How a call's work is split.  256-tiles where they use the chip: the outputs they cover take at
 // least kFill of the 256 CUs' whole passes (a tile per CU and pass), ragged edges and a last pass
 // that is partly empty counted as lost; else 128-tiles, whose two workgroups per CU hide each
-// other's epilogues.  Measured (256 / 128): N 509, V 32000, d 768 (fills 0.97 / 0.73 / -) S^T 34.4 /
-// 37.3 us, grad_W 42.6 / 35.9 us; N 4096, d 1024 (0.98) both directions together 1149 / 1220 us.
+// other's epilogues.  Measured per product (fill: 256 / 128 us), S^T of the forward: 0.49: 33.6 / 28.4, 0.54: 34.6 /
+// 31.8, 0.73: 57.5 / 51.0, 0.75: 68.3 / 71.1, 0.89: 59.1 / 66.9, 0.97: 33.5 / 37.1, 0.98 (N 4096, V 32000,
+// d 1024): 306 / 336; grad_W: 0.42: 50.8 / 32.2, 0.73: 42.8 / 35.0, 54.6 / 46.3 and (N 4096) 107 / 115, 0.80: 26.6
+// / 28.2, 0.98: 45.4 / 44.3 (N 512) and 253 / 304 (N 4096).  grad_h, whose tiles are split over K, by
+// its tiles of 256: 8: 47.8 / 43.5, 16: 77.6 / 77.3, 24: 106 / 116 and 42.6 / 36.3, 32: 133 / 147, 64: 259 / 340.
 struct Plan {
   int Np;          // tokens padded to 256
   int C;           // vocabulary ids per chunk (a multiple of 256)
