@@ -11,7 +11,8 @@
  *                      <- the chunk buffers of the reference's loops (model.py:293-301, 344-353)
  *
  * Shapes: h (n_rows, d_model) bf16 row-major, weight (vocab, d_model) bf16 row-major, targets
- * int32 (n_rows).  d_model a multiple of 128, n_rows and vocab >= 1.  Every logit is a bf16 x bf16
+ * int32 (n_rows).  d_model a multiple of 128, n_rows and vocab >= 1; h, weight, the workspace and the
+ * gradients 16-byte aligned (they move in 16-byte pieces).  Every logit is a bf16 x bf16
  * dot product accumulated in f32 on the matrix cores; the softmax statistics are f32.
  * All calls are asynchronous on `stream` (a hipStream_t) and return MSD_OK or a negative
  * MSD_E_* code (msdecode.h); a target id outside [0, vocab) is replaced by 0 and reported as bit 2

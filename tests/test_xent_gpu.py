@@ -131,6 +131,21 @@ def test_deterministic_and_3d_wrapper():
     assert np.array_equal(gw.float().cpu().numpy(), a[2])
 
 
+def test_operands_off_a_16_byte_boundary():
+    """Slices of a flat buffer at any offset give the bits of aligned tensors."""
+    h, w, t = _inputs(130, 700, 256, seed=9)
+    want = _run(h, w, t, 512)
+    for off in (1, 4):
+        flat = torch.empty(off + h.numel() + w.numel(), dtype=torch.bfloat16, device="cuda")
+        hd = flat[off:off + h.numel()].view_as(h).copy_(h.cuda()).requires_grad_()
+        wd = flat[off + h.numel():].view_as(w).copy_(w.cuda()).requires_grad_()
+        assert hd.data_ptr() % 16 and wd.data_ptr() % 16
+        loss = fused_cross_entropy(hd, wd, t.cuda(), 512)
+        gh, gw = torch.autograd.grad(loss, (hd, wd))
+        assert float(loss) == want[0]
+        assert np.array_equal(gh.float().cpu().numpy(), want[1]) and np.array_equal(gw.float().cpu().numpy(), want[2])
+
+
 def _loss_and_grads(x, check):
     h, w, t = x
     loss = fused_cross_entropy(h, w, t, 512, check_targets=check)

@@ -42,6 +42,13 @@ def _workspace(like, n, V, d, chunk):
     return like.new_empty(_workspace_bytes(n, V, d, chunk), dtype=torch.uint8)
 
 
+def _operand(x):
+    """x in row-major order on a 16-byte boundary, which the kernels' loads take (a slice of a flat parameter
+    buffer may start anywhere)."""
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def _row_pointers(rows, n):
     p = rows.data_ptr()
     return p, p + 4 * n, p + 4 * n + 4
@@ -66,7 +73,7 @@ class FusedCrossEntropy(torch.autograd.Function):
     @staticmethod
     def forward(ctx, h, weight, targets, chunk_size, check_targets):
         _check_inputs(h, weight, targets)
-        h, weight = h.contiguous(), weight.contiguous()
+        h, weight = _operand(h), _operand(weight)
         N, d = h.shape
         V = weight.shape[0]
         chunk = int(chunk_size)
